@@ -115,6 +115,7 @@ __device__ __forceinline__ void write_base_grad(const PreprocessBackwardArgs& a,
 // 2D mean / conic / opacity gradients through the projection to the 3D mean, log-scales and quaternion
 __device__ inline void geometry_backward(const PreprocessBackwardArgs& a, uint32_t p, const PrimRecord& rec, const GeometryInputs& gi,
                                          const InstanceGrads& ig, float3 dmean_color) {
+#pragma clang fp contract(fast)  // (gradients decide nothing: sums and products fused)
     const float3 mean = gi.mean;
     const float gmx = ig.gmx, gmy = ig.gmy;
     const float3 gconic = make_float3(ig.gcx, ig.gcy, ig.gcz);
