@@ -7,26 +7,40 @@ namespace efgs {
 
 constexpr float sv_eps = 1e-12f;
 
-template <int RES_ACT>
-__device__ inline float3 sv_residual(const float* p, float3 d, uint32_t sites) {
-    if (sites == 0) return make_float3(0.0f, 0.0f, 0.0f);
+// running softmax over the sites
+struct SvState {
     float max_logit = -1e30f, wsum = 0.0f, r = 0.0f, g = 0.0f, b = 0.0f;
+};
+
+template <int RES_ACT>
+__device__ __forceinline__ void sv_add_sites(SvState& v, const float* p, float3 d, uint32_t sites) {
     for (uint32_t s = 0; s < sites; s++, p += 7) {
         const float inv = 1.0f / fmaxf(sqrtf(p[0] * p[0] + p[1] * p[1] + p[2] * p[2]), sv_eps);
         const float d0 = inv * p[0] - d.x, d1 = inv * p[1] - d.y, d2 = inv * p[2] - d.z;
         const float dist = sqrtf(d0 * d0 + d1 * d1 + d2 * d2);
         const float logit = -expf(p[3]) * dist;
-        const float nm = fmaxf(max_logit, logit);
-        const float rescale = expf(max_logit - nm);
+        const float nm = fmaxf(v.max_logit, logit);
+        const float rescale = expf(v.max_logit - nm);
         const float w = expf(fminf(logit - nm, 0.0f));
-        wsum = wsum * rescale + w;
-        r = r * rescale + w * residual_activation<RES_ACT>(p[4]);
-        g = g * rescale + w * residual_activation<RES_ACT>(p[5]);
-        b = b * rescale + w * residual_activation<RES_ACT>(p[6]);
-        max_logit = nm;
+        v.wsum = v.wsum * rescale + w;
+        v.r = v.r * rescale + w * residual_activation<RES_ACT>(p[4]);
+        v.g = v.g * rescale + w * residual_activation<RES_ACT>(p[5]);
+        v.b = v.b * rescale + w * residual_activation<RES_ACT>(p[6]);
+        v.max_logit = nm;
     }
-    const float wr = 1.0f / wsum;
-    return make_float3(wr * r, wr * g, wr * b);
+}
+
+__device__ __forceinline__ float3 sv_color(const SvState& v) {
+    const float wr = 1.0f / v.wsum;
+    return make_float3(wr * v.r, wr * v.g, wr * v.b);
+}
+
+template <int RES_ACT>
+__device__ inline float3 sv_residual(const float* p, float3 d, uint32_t sites) {
+    if (sites == 0) return make_float3(0.0f, 0.0f, 0.0f);
+    SvState v;
+    sv_add_sites<RES_ACT>(v, p, d, sites);
+    return sv_color(v);
 }
 
 // writes dL/d(site parameters) of the active sites and returns dL/dmean through the view direction. A site's

@@ -251,8 +251,11 @@ extern "C" __global__ __launch_bounds__(efgs::backward_block) void EFGS_KERNEL_N
 #if EFGS_MODEL != 0
     if constexpr (BackwardRows::staged) {
         constexpr uint32_t row_ld = BackwardRows::row_ld, pass_units = BackwardRows::pass_units, n_passes = BackwardRows::n_passes;
-        __shared__ float s_rows[backward_block * row_ld];
-        const uint32_t p0 = blockIdx.x * backward_block, p = p0 + threadIdx.x;
+        __shared__ float s_rows[(backward_block / 64) * BackwardRows::wave_floats];
+        const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        float* const rows = s_rows + wave * BackwardRows::wave_floats;
+        float* const row = rows + lane * row_ld;
+        const uint32_t p0 = blockIdx.x * backward_block + wave * 64u, p = p0 + lane;
         const bool active = p < a.n;
         const uint32_t touched = active ? a.n_touched[p] : 0u;
         const uint32_t offset = active ? a.prim_offset[p] : 0u;
@@ -271,18 +274,18 @@ extern "C" __global__ __launch_bounds__(efgs::backward_block) void EFGS_KERNEL_N
             const float3 cam = make_float3(a.cam.cam_position[0], a.cam.cam_position[1], a.cam.cam_position[2]);
             d = view_direction(gi.mean, cam, norm_rcp);
         }
-        const uint32_t rows = p0 < a.n ? min(backward_block, a.n - p0) : 0u;
+        const uint32_t n_rows = p0 < a.n ? min(64u, a.n - p0) : 0u;
+        const uint64_t work_mask = __ballot(work);
         for (uint32_t pass = 0; pass < n_passes; pass++) {
             const uint32_t u0 = pass * pass_units;
             const uint32_t nu = min(pass_units, static_cast<uint32_t>(EFGS_N_UNITS) - u0);
-            if (pass > 0) __syncthreads();  // every thread has read the previous pass's rows
-            stage_residual_rows<backward_block, row_ld>(a.residual, p0, rows, u0 * params_per_unit, nu * params_per_unit, s_rows);
-            __syncthreads();
+            // the gradients replace the staged row in place (each parameter is read before its gradient is written) and
+            // leave with coalesced stores; the units past the active degree and the rows of primitives without
+            // instances get zeros
+            if (pass > 0) rows_sync();  // the previous pass's gradients have been read
 #if EFGS_MODEL == 1 || EFGS_MODEL == 2
-            // (one pass: every coefficient / site of the row) the gradients replace the staged row in place (each
-            // parameter is read before its gradient is written) and leave with coalesced stores; the units past the
-            // active degree and the rows of primitives without instances get zeros
-            float* row = s_rows + threadIdx.x * row_ld;
+            const uint32_t n_active = work ? active_residual_params(a.cam.degree) : 0u;  // (one pass: the whole row)
+            stage_rows<row_ld>(a.residual, p0, a.cam.degree > 0 ? work_mask : 0ull, 0u, residual_params, rows);
             if (work) {
 #if EFGS_MODEL == 1
                 dmean_color = sh_residual_backward<EFGS_RES_ACT>(row, dpre, row, d, norm_rcp, a.cam.degree);
@@ -290,25 +293,19 @@ extern "C" __global__ __launch_bounds__(efgs::backward_block) void EFGS_KERNEL_N
                 dmean_color = sv_residual_backward<EFGS_RES_ACT>(row, dpre, row, d, norm_rcp, a.cam.degree);
 #endif
             }
-            for (uint32_t i = work ? active_residual_params(a.cam.degree) : 0u; i < residual_params; i++) row[i] = 0.0f;
-            __syncthreads();
-            store_residual_rows<backward_block, row_ld>(s_rows, p0, rows, 0u, residual_params, a.g_residual);
 #else
-            // lobes: a lobe's parameters are read before its gradients are written, so the gradients replace the
-            // staged row in place (zero for inactive lobes and for primitives without instances) and leave with
-            // coalesced stores
-            float* row = s_rows + threadIdx.x * row_ld;
-            const uint32_t na = work && a.cam.degree > u0 ? min(nu, a.cam.degree - u0) : 0u;
+            const uint32_t na = a.cam.degree > u0 ? min(nu, a.cam.degree - u0) : 0u;
+            const uint32_t n_active = work ? na * params_per_unit : 0u;
+            stage_rows<row_ld>(a.residual, p0, na > 0 ? work_mask : 0ull, u0 * params_per_unit, nu * params_per_unit, rows);
             if (work) {
                 const float3 dm = lobe_residual_backward<EFGS_RES_ACT, EFGS_MODEL == 4>(row, dpre, row, d, norm_rcp, na);
                 dmean_color.x += dm.x;
                 dmean_color.y += dm.y;
                 dmean_color.z += dm.z;
             }
-            for (uint32_t i = na * params_per_unit; i < nu * params_per_unit; i++) row[i] = 0.0f;
-            __syncthreads();
-            store_residual_rows<backward_block, row_ld>(s_rows, p0, rows, u0 * params_per_unit, nu * params_per_unit, a.g_residual);
 #endif
+            for (uint32_t i = n_active; i < nu * params_per_unit; i++) row[i] = 0.0f;
+            store_rows<row_ld>(rows, p0, n_rows, u0 * params_per_unit, nu * params_per_unit, a.g_residual);
         }
         if (work) {
             geometry_backward(a, p, rec, gi, ig, dmean_color);

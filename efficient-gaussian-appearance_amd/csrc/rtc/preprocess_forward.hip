@@ -180,11 +180,10 @@ extern "C" __global__ __launch_bounds__(256, 4) void EFGS_KERNEL_NAME(efgs::Prep
     const uint32_t wave = threadIdx.x >> 6;
     __shared__ uint32_t wave_counts[4 * (preprocess_block / 64)];
 #if EFGS_MODEL >= 1 && EFGS_MODEL <= 4
-    // the forward stages its rows only for the lobe models: SH and SV read each row once and keep more waves per
-    // SIMD without the LDS
-    constexpr bool staged_forward = ForwardRows::staged && (EFGS_MODEL == 3 || EFGS_MODEL == 4);
     constexpr uint32_t row_ld = ForwardRows::row_ld, pass_units = ForwardRows::pass_units, n_passes = ForwardRows::n_passes;
-    __shared__ float s_rows[staged_forward ? preprocess_block * row_ld : 1];
+    __shared__ float s_rows[(preprocess_block / 64) * ForwardRows::wave_floats];
+    const uint32_t wave_u = __builtin_amdgcn_readfirstlane(wave);
+    float* const rows = s_rows + wave_u * ForwardRows::wave_floats;
 #endif
 #if EFGS_MODEL == 5
     // residual MLP weights staged once per block (padded rows); staging rows of the MLP inputs (64 per wave)
@@ -281,31 +280,34 @@ extern "C" __global__ __launch_bounds__(256, 4) void EFGS_KERNEL_NAME(efgs::Prep
         }
 #endif
 #if EFGS_MODEL >= 1 && EFGS_MODEL <= 4
-        if constexpr (staged_forward) {
-            // the chunk's rows through LDS (the previous chunk ended at a block barrier), one pass per unit range
-            const uint32_t p0 = chunk * preprocess_block;
-            const uint32_t rows = min(preprocess_block, a.n - p0);
+        if constexpr (ForwardRows::staged) {
+            const uint32_t p0 = chunk * preprocess_block + wave_u * 64u;
+            const float* const row = rows + lane * row_ld;
+#if EFGS_MODEL == 2
+            SvState sv;
+#endif
             for (uint32_t pass = 0; pass < n_passes; pass++) {
                 const uint32_t u0 = pass * pass_units;
+                if (u0 >= a.cam.degree && EFGS_MODEL != 1) break;  // (uniform: no active unit is left)
                 const uint32_t nu = min(pass_units, static_cast<uint32_t>(EFGS_N_UNITS) - u0);
-                if (pass > 0) __syncthreads();  // every thread has read the previous pass's rows
-                stage_residual_rows<preprocess_block, row_ld>(a.residual, p0, rows, u0 * params_per_unit, nu * params_per_unit, s_rows);
-                __syncthreads();
+                rows_sync();  // every lane has read the previous rows
+                stage_rows<row_ld>(a.residual, p0, a.cam.degree > 0 ? visible_mask : 0ull, u0 * params_per_unit, nu * params_per_unit, rows);
                 if (visible) {
-                    const float* row = s_rows + threadIdx.x * row_ld;
 #if EFGS_MODEL == 1
                     res = sh_residual<EFGS_RES_ACT>(row, d, a.cam.degree);
 #elif EFGS_MODEL == 2
-                    res = sv_residual<EFGS_RES_ACT>(row, d, a.cam.degree);
+                    sv_add_sites<EFGS_RES_ACT>(sv, row, d, min(nu, a.cam.degree - u0));
 #else
-                    const uint32_t na = a.cam.degree > u0 ? min(nu, a.cam.degree - u0) : 0u;
-                    const float3 r = lobe_residual<EFGS_RES_ACT, EFGS_MODEL == 4>(row, d, na);
+                    const float3 r = lobe_residual<EFGS_RES_ACT, EFGS_MODEL == 4>(row, d, min(nu, a.cam.degree - u0));
                     res.x += r.x;
                     res.y += r.y;
                     res.z += r.z;
 #endif
                 }
             }
+#if EFGS_MODEL == 2
+            if (visible && a.cam.degree > 0) res = sv_color(sv);
+#endif
         } else if (visible) {
 #if EFGS_MODEL == 1
             res = sh_residual<EFGS_RES_ACT>(rp, d, a.cam.degree);

@@ -1,4 +1,4 @@
-// Per-primitive residual parameters of the preprocess kernels: their count and the LDS staging of a block's rows.
+// Per-primitive residual parameters of the preprocess kernels: their count and the LDS staging of a wave's rows.
 #pragma once
 
 namespace efgs {
@@ -7,57 +7,61 @@ namespace efgs {
 constexpr uint32_t params_per_unit = EFGS_MODEL == 1 ? 3u : EFGS_MODEL == 2 ? 7u : EFGS_MODEL == 3 ? 8u : EFGS_MODEL == 4 ? 9u : 1u;
 constexpr uint32_t residual_params = EFGS_MODEL == 0 ? 0u : params_per_unit * EFGS_N_UNITS;
 
-// Residual rows of a block staged through LDS with coalesced loads (a thread's own row is 45-72 floats apart from
-// its neighbours', so direct per-thread reads spread every load instruction of a wave over 64 cache lines). Whole
-// units per pass: SH (coefficients) and SV (sites: the backward's softmax needs them all) in one pass, lobes in
-// passes of at most MAX_FLOATS floats; a layout that does not fit reads its rows directly. Fewer floats per pass
-// mean less LDS per block and more waves per SIMD, at one barrier and one staging round more per pass (the SV
-// forward in passes of two sites, its softmax carried online, measured 105 -> 131 us: it stays unstaged): the lobe
-// forward runs best at 18 (2 lobes per pass; NASG 149 -> 119 us, NASGabor 233 -> 162 us on 1M Gaussians against
-// 40), the lobe backward, which also writes its gradients back through the rows, at 40 (24: 221 -> 310 us).
-template <uint32_t MAX_FLOATS>
+// A wave stages its 64 primitives' residual rows in its own part of the LDS, whole units per pass: a thread's own row
+// is 45-72 floats apart from its neighbours', so direct per-thread reads touch 64 cache lines per load instruction and
+// a wave's lines fall out of the L1 and the L2 between the loads that share them (400k SH3 primitives: 271 MB read
+// for 94 MB of rows). SH takes its coefficients in one pass, SV and the lobe models up to MAX_UNITS units per pass:
+// four lobes are 128 (144) bytes of a row, where passes of two lobes fetched every 128-byte line twice (NASG forward on
+// 1M primitives: 488 MB for 312 MB). A layout above 63 floats per pass (WHOLE_ROW: per row) reads its rows directly.
+// Preprocess times before and after (the block-wide staging, respectively direct reads, of single floats with index
+// arithmetic per element): NASG on 1M at 1080p 120 -> 90 us forward, 181 -> 142 us backward; SH3 on 400k 66 -> 36 us
+// forward; SV on 150k 31.0 -> 30.6 and 37.9 -> 35.0 us.
+template <uint32_t MAX_UNITS, bool WHOLE_ROW>
 struct RowStaging {
-    static constexpr uint32_t max_floats = EFGS_MODEL == 1 || EFGS_MODEL == 2 ? 63u : MAX_FLOATS;
-    static constexpr uint32_t units_fit = params_per_unit > 0 ? max_floats / params_per_unit : 0u;
-    static constexpr uint32_t pass_units = EFGS_MODEL == 1 || EFGS_MODEL == 2 ? EFGS_N_UNITS
-                                                                               : (units_fit < EFGS_N_UNITS ? units_fit : EFGS_N_UNITS);
-    static constexpr bool staged = EFGS_MODEL != 0 && EFGS_N_UNITS > 0 && pass_units > 0 && pass_units * params_per_unit <= max_floats;
-    static constexpr uint32_t row_ld = (pass_units * params_per_unit) | 1u;
+    static constexpr uint32_t pass_units = EFGS_MODEL == 1 ? EFGS_N_UNITS : (MAX_UNITS < EFGS_N_UNITS ? MAX_UNITS : EFGS_N_UNITS);
+    static constexpr uint32_t pass_floats = pass_units * params_per_unit;
+    static constexpr bool staged = EFGS_MODEL != 0 && EFGS_MODEL != 5 && EFGS_N_UNITS > 0 && pass_floats <= 63u &&
+                                   (!WHOLE_ROW || pass_units == EFGS_N_UNITS);
+    static constexpr uint32_t row_ld = pass_floats | 1u;  // odd: the lanes' rows start in different banks
     static constexpr uint32_t n_passes = pass_units > 0 ? (EFGS_N_UNITS + pass_units - 1) / pass_units : 0u;
+    static constexpr uint32_t wave_floats = staged ? 64u * row_ld : 1u;
 };
-using ForwardRows = RowStaging<18u>;
-using BackwardRows = RowStaging<40u>;
+using ForwardRows = RowStaging<4u, false>;
+using BackwardRows = RowStaging<EFGS_MODEL == 2 ? 9u : 4u, EFGS_MODEL == 2>;  // (the SV backward's softmax needs every site)
 
-// rows [p0, p0 + rows), floats [f0, f0 + floats) of each, into s[r * ROW_LD + c] by the BLOCK threads of the block;
-// (r, c) advance by (BLOCK / floats, BLOCK % floats) per step, eight loads in flight
-template <uint32_t BLOCK, uint32_t ROW_LD>
-__device__ __forceinline__ void stage_residual_rows(const float* residual, uint32_t p0, uint32_t rows, uint32_t f0, uint32_t floats, float* s) {
-    const uint32_t total = rows * floats, dr = BLOCK / floats, dc = BLOCK - dr * floats;
-    uint32_t r = threadIdx.x / floats, c = threadIdx.x - r * floats;
-#pragma unroll 8
-    for (uint32_t i = threadIdx.x; i < total; i += BLOCK) {
-        s[r * ROW_LD + c] = residual[static_cast<size_t>(p0 + r) * residual_params + f0 + c];
-        c += dc;
-        r += dr;
-        const bool wrap = c >= floats;
-        c = wrap ? c - floats : c;
-        r = wrap ? r + 1 : r;
-    }
+__device__ __forceinline__ void rows_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// the reverse of stage_residual_rows: s[r * ROW_LD + c] to rows [p0, p0 + rows), floats [f0, f0 + floats) of `out`
-template <uint32_t BLOCK, uint32_t ROW_LD>
-__device__ __forceinline__ void store_residual_rows(const float* s, uint32_t p0, uint32_t rows, uint32_t f0, uint32_t floats, float* out) {
-    const uint32_t total = rows * floats, dr = BLOCK / floats, dc = BLOCK - dr * floats;
-    uint32_t r = threadIdx.x / floats, c = threadIdx.x - r * floats;
+// The rows in `mask` (bit r: primitive p0 + r; p0 and mask wave-uniform) from `residual` into s[r * ROW_LD + c], floats
+// [f0, f0 + floats) of each (floats <= 64): one load instruction per row straight into the LDS (no registers, no
+// per-element index arithmetic), all in flight together; returns when they have landed.
+template <uint32_t ROW_LD>
+__device__ __forceinline__ void stage_rows(const float* residual, uint32_t p0, uint64_t mask, uint32_t f0, uint32_t floats, float* s) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const float* const base = residual + static_cast<size_t>(p0) * residual_params + f0;
+    if (lane < floats) {
+        for (uint64_t m = mask; m != 0; m &= m - 1) {
+            const uint32_t r = static_cast<uint32_t>(__ffsll(static_cast<long long>(m)) - 1);
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(base + r * residual_params + lane),
+                                             (__attribute__((address_space(3))) void*)(s + r * ROW_LD), 4, 0, 0);
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    rows_sync();
+}
+
+// the reverse of stage_rows for rows [0, rows): s[r * ROW_LD + c] to floats [f0, f0 + floats) of primitive p0 + r
+template <uint32_t ROW_LD>
+__device__ __forceinline__ void store_rows(const float* s, uint32_t p0, uint32_t rows, uint32_t f0, uint32_t floats, float* out) {
+    const uint32_t lane = threadIdx.x & 63u;
+    rows_sync();
+    float* const base = out + static_cast<size_t>(p0) * residual_params + f0;
+    if (lane < floats) {
 #pragma unroll 8
-    for (uint32_t i = threadIdx.x; i < total; i += BLOCK) {
-        out[static_cast<size_t>(p0 + r) * residual_params + f0 + c] = s[r * ROW_LD + c];
-        c += dc;
-        r += dr;
-        const bool wrap = c >= floats;
-        c = wrap ? c - floats : c;
-        r = wrap ? r + 1 : r;
+        for (uint32_t r = 0; r < rows; r++) base[r * residual_params + lane] = s[r * ROW_LD + lane];
     }
 }
 
