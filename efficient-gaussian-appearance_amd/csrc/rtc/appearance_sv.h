@@ -6,6 +6,39 @@
 namespace efgs {
 
 constexpr float sv_eps = 1e-12f;
+constexpr float sv_log2e = 1.44269504088896340736f, sv_ln2 = 0.69314718055994530942f;
+
+// Site arithmetic on the hardware's exp2, reciprocal (square root) and square root (1 ulp each) and fused
+// multiply-adds; the softmax runs on base-2 logits, one exponential per site (the larger of the running maximum and the
+// new logit has weight 1). Colours and gradients are as close to 64-bit results as with the library's exp and correctly
+// rounded divides and square roots, which were most of a site's instructions.
+
+// exp x with the rounding of x log2 e compensated (x clamped to the range of finite, normal results; NaN: the largest)
+__device__ __forceinline__ float sv_exp(float x) {
+    x = fmaxf(fminf(x, 88.0f), -87.0f);
+    const float t = x * sv_log2e;
+    const float r = __builtin_fmaf(x, 1.92596299e-8f, __builtin_fmaf(x, sv_log2e, -t));
+    const float e = __builtin_amdgcn_exp2f(t);
+    return __builtin_fmaf(e, r * sv_ln2, e);
+}
+
+__device__ __forceinline__ float sv_dot(float x, float y, float z) { return __builtin_fmaf(z, z, __builtin_fmaf(y, y, x * x)); }
+
+// a site: its unit direction minus the view direction, their distance, its sharpness and the base-2 logit
+struct SvSite {
+    float inv, dx, dy, dz, dist, tau, logit;
+};
+__device__ __forceinline__ SvSite sv_site(const float* p, float3 d) {
+    SvSite s;
+    s.inv = __builtin_amdgcn_rsqf(fmaxf(sv_dot(p[0], p[1], p[2]), sv_eps * sv_eps));
+    s.dx = __builtin_fmaf(s.inv, p[0], -d.x);
+    s.dy = __builtin_fmaf(s.inv, p[1], -d.y);
+    s.dz = __builtin_fmaf(s.inv, p[2], -d.z);
+    s.dist = __builtin_amdgcn_sqrtf(sv_dot(s.dx, s.dy, s.dz));
+    s.tau = sv_exp(p[3]);
+    s.logit = -(s.tau * sv_log2e) * s.dist;
+    return s;
+}
 
 // running softmax over the sites
 struct SvState {
@@ -15,23 +48,20 @@ struct SvState {
 template <int RES_ACT>
 __device__ __forceinline__ void sv_add_sites(SvState& v, const float* p, float3 d, uint32_t sites) {
     for (uint32_t s = 0; s < sites; s++, p += 7) {
-        const float inv = 1.0f / fmaxf(sqrtf(p[0] * p[0] + p[1] * p[1] + p[2] * p[2]), sv_eps);
-        const float d0 = inv * p[0] - d.x, d1 = inv * p[1] - d.y, d2 = inv * p[2] - d.z;
-        const float dist = sqrtf(d0 * d0 + d1 * d1 + d2 * d2);
-        const float logit = -expf(p[3]) * dist;
-        const float nm = fmaxf(v.max_logit, logit);
-        const float rescale = expf(v.max_logit - nm);
-        const float w = expf(fminf(logit - nm, 0.0f));
-        v.wsum = v.wsum * rescale + w;
-        v.r = v.r * rescale + w * residual_activation<RES_ACT>(p[4]);
-        v.g = v.g * rescale + w * residual_activation<RES_ACT>(p[5]);
-        v.b = v.b * rescale + w * residual_activation<RES_ACT>(p[6]);
-        v.max_logit = nm;
+        const float logit = sv_site(p, d).logit;
+        const bool higher = logit > v.max_logit;
+        const float e = __builtin_amdgcn_exp2f(fminf(-fabsf(logit - v.max_logit), 0.0f));  // (NaN: 1)
+        const float rescale = higher ? e : 1.0f, w = higher ? 1.0f : e;
+        v.wsum = __builtin_fmaf(v.wsum, rescale, w);
+        v.r = __builtin_fmaf(v.r, rescale, w * residual_activation<RES_ACT>(p[4]));
+        v.g = __builtin_fmaf(v.g, rescale, w * residual_activation<RES_ACT>(p[5]));
+        v.b = __builtin_fmaf(v.b, rescale, w * residual_activation<RES_ACT>(p[6]));
+        v.max_logit = higher ? logit : v.max_logit;
     }
 }
 
 __device__ __forceinline__ float3 sv_color(const SvState& v) {
-    const float wr = 1.0f / v.wsum;
+    const float wr = __builtin_amdgcn_rcpf(v.wsum);
     return make_float3(wr * v.r, wr * v.g, wr * v.b);
 }
 
@@ -47,51 +77,35 @@ __device__ inline float3 sv_residual(const float* p, float3 d, uint32_t sites) {
 // parameters are read before its gradients are written, and no later step reads them, so gp may be p0 itself.
 template <int RES_ACT>
 __device__ inline float3 sv_residual_backward(const float* p0, float3 gc, float* gp, float3 d, float norm_rcp, uint32_t sites) {
+#pragma clang fp contract(fast)
     if (sites == 0) return make_float3(0.0f, 0.0f, 0.0f);
-    float max_logit = -1e30f, wsum = 0.0f, r = 0.0f, g = 0.0f, b = 0.0f;
-    const float* p = p0;
-    for (uint32_t s = 0; s < sites; s++, p += 7) {
-        const float inv = 1.0f / fmaxf(sqrtf(p[0] * p[0] + p[1] * p[1] + p[2] * p[2]), sv_eps);
-        const float d0 = inv * p[0] - d.x, d1 = inv * p[1] - d.y, d2 = inv * p[2] - d.z;
-        const float dist = sqrtf(d0 * d0 + d1 * d1 + d2 * d2);
-        const float logit = -expf(p[3]) * dist;
-        const float nm = fmaxf(max_logit, logit);
-        const float rescale = expf(max_logit - nm);
-        const float w = expf(fminf(logit - nm, 0.0f));
-        wsum = wsum * rescale + w;
-        r = r * rescale + w * residual_activation<RES_ACT>(p[4]);
-        g = g * rescale + w * residual_activation<RES_ACT>(p[5]);
-        b = b * rescale + w * residual_activation<RES_ACT>(p[6]);
-        max_logit = nm;
-    }
-    const float wr = 1.0f / wsum;
-    const float gmean = gc.x * (wr * r) + gc.y * (wr * g) + gc.z * (wr * b);
+    SvState v;
+    sv_add_sites<RES_ACT>(v, p0, d, sites);
+    const float wr = __builtin_amdgcn_rcpf(v.wsum);
+    const float gmean = wr * (gc.x * v.r + gc.y * v.g + gc.z * v.b);
     float3 gd = make_float3(0.0f, 0.0f, 0.0f);
-    p = p0;
+    const float* p = p0;
     for (uint32_t s = 0; s < sites; s++, p += 7, gp += 7) {
-        const float lr = 1.0f / fmaxf(sqrtf(p[0] * p[0] + p[1] * p[1] + p[2] * p[2]), sv_eps);
-        const float3 site = make_float3(lr * p[0], lr * p[1], lr * p[2]);
-        const float3 sd = make_float3(site.x - d.x, site.y - d.y, site.z - d.z);
-        const float dist = sqrtf(sd.x * sd.x + sd.y * sd.y + sd.z * sd.z);
-        const float tau = expf(p[3]);
-        const float w = expf(fminf(-tau * dist - max_logit, 0.0f)) * wr;
+        const SvSite q = sv_site(p, d);
+        const float w = __builtin_amdgcn_exp2f(fminf(q.logit - v.max_logit, 0.0f)) * wr;
         const float cr = residual_activation<RES_ACT>(p[4]);
         const float cg = residual_activation<RES_ACT>(p[5]);
         const float cb = residual_activation<RES_ACT>(p[6]);
+        const float3 site = make_float3(q.inv * p[0], q.inv * p[1], q.inv * p[2]);
         gp[4] = w * gc.x * residual_activation_grad<RES_ACT>(cr);
         gp[5] = w * gc.y * residual_activation_grad<RES_ACT>(cg);
         gp[6] = w * gc.z * residual_activation_grad<RES_ACT>(cb);
         const float glogit = w * ((gc.x * cr + gc.y * cg + gc.z * cb) - gmean);
-        gp[3] = -dist * tau * glogit;
-        const float f = (-tau * glogit) / fmaxf(dist, sv_eps);
-        const float3 gsd = make_float3(f * sd.x, f * sd.y, f * sd.z);
-        const float dd = gsd.x * site.x + gsd.y * site.y + gsd.z * site.z;
-        gp[0] = (gsd.x - dd * site.x) * lr;
-        gp[1] = (gsd.y - dd * site.y) * lr;
-        gp[2] = (gsd.z - dd * site.z) * lr;
-        gd.x -= gsd.x;
-        gd.y -= gsd.y;
-        gd.z -= gsd.z;
+        gp[3] = -q.dist * q.tau * glogit;
+        const float f = -q.tau * glogit * __builtin_amdgcn_rcpf(fmaxf(q.dist, sv_eps));
+        const float gx = f * q.dx, gy = f * q.dy, gz = f * q.dz;
+        const float dd = gx * site.x + gy * site.y + gz * site.z;
+        gp[0] = (gx - dd * site.x) * q.inv;
+        gp[1] = (gy - dd * site.y) * q.inv;
+        gp[2] = (gz - dd * site.z) * q.inv;
+        gd.x -= gx;
+        gd.y -= gy;
+        gd.z -= gz;
     }
     return direction_grad_to_mean(gd, d, norm_rcp);
 }
