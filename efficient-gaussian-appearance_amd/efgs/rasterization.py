@@ -1,17 +1,16 @@
 """Python interface of the rasterizer, mirroring the reference bindings
 (FasterGSVDACudaBackend/FasterGSVDACudaBackend/torch_bindings/rasterization.py:1-251): same function names,
-argument meaning and error behaviour, backed by libefgs_hip.so through ctypes.
+argument meaning and error behaviour, backed by libefgs_hip.so: the differentiable functions through the C++ autograd
+functions of csrc/torch_binding.cpp (_native), the others through ctypes.
 """
 from __future__ import annotations
 
-import contextlib
 import ctypes
 from typing import Any, NamedTuple
 
 import torch
-from torch.autograd.function import once_differentiable
 
-from . import _lib
+from . import _lib, _native
 from ._lib import check, lib
 
 APPEARANCE_MODEL_IDS = {'sh': 1, 'sv': 2, 'nasg': 3, 'nasgabor': 4, 'neural': 5}  # 0: internal precomputed-colour variant
@@ -180,16 +179,11 @@ def _check_inputs(means, scales, rotations, opacities, precomputed_colors, base_
     return device
 
 
-def _forward(means, scales, rotations, opacities, precomputed_colors, base_colors, residual_params, mlp_weights_f32, settings,
-             native=None):
-    """native: (settings struct, tensors it points to, primitives struct) already built for these inputs, or None."""
+def _forward(means, scales, rotations, opacities, precomputed_colors, base_colors, residual_params, mlp_weights_f32, settings):
     device = _check_inputs(means, scales, rotations, opacities, precomputed_colors, base_colors, residual_params, mlp_weights_f32)
     with torch.cuda.device(device):
-        if native is not None:
-            cs, keep, prims = native
-        else:
-            cs, keep = _native_settings(settings, device)
-            prims = _native_primitives(means, scales, rotations, opacities, precomputed_colors, base_colors, residual_params, mlp_weights_f32)
+        cs, keep = _native_settings(settings, device)
+        prims = _native_primitives(means, scales, rotations, opacities, precomputed_colors, base_colors, residual_params, mlp_weights_f32)
         image = torch.empty((3, int(settings.height), int(settings.width)), dtype=torch.float32, device=device)
         alloc = _lib.WorkspaceAllocator(device, 'forward')
         frame = _lib.Frame()
@@ -201,100 +195,6 @@ def _forward(means, scales, rotations, opacities, precomputed_colors, base_color
     return image, frame, alloc.tensors, keep
 
 
-class _Rasterize(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx: Any, means, scales, rotations, opacities, precomputed_colors, base_colors, residual_params, mlp_weights,
-                densification_info, rasterizer_settings: RasterizerSettings) -> torch.Tensor:
-        mlp_weights_f32 = mlp_weights.detach().float().contiguous() if mlp_weights.numel() > 0 else torch.empty(0, dtype=torch.float32, device=means.device)
-        ctx.mlp_numel = mlp_weights.numel()
-        # the backward's host-side state is built before the forward launches anything: the host is then still ahead
-        # of the GPU (which runs the previous work), and between the forward's counter read and the backward's first
-        # launch only autograd's own bookkeeping runs on the host while the GPU finishes the binning and the blend
-        prep = _prepare_backward(ctx, means, scales, rotations, opacities, precomputed_colors, base_colors, residual_params,
-                                 mlp_weights_f32, densification_info, rasterizer_settings) if any(ctx.needs_input_grad) else None
-        ctx.prepared = prep
-        image, frame, buffers, _ = _forward(means, scales, rotations, opacities, precomputed_colors, base_colors, residual_params,
-                                            mlp_weights_f32, rasterizer_settings,
-                                            native=(prep.settings, prep.keep, prep.prims) if prep is not None else None)
-        ctx.rasterizer_settings = rasterizer_settings
-        ctx.frame = frame
-        ctx.buffers = buffers
-        ctx.save_for_backward(image, means, scales, rotations, opacities, precomputed_colors, base_colors, residual_params, mlp_weights_f32)
-        ctx.densification_info = densification_info
-        ctx.mark_non_differentiable(densification_info)
-        return image
-
-    @staticmethod
-    @once_differentiable
-    def backward(ctx: Any, grad_image: torch.Tensor):
-        saved = ctx.saved_tensors  # unpacking checks that no saved tensor was modified in place
-        image = saved[0]
-        # a second backward of the same graph (retain_graph) gets fresh outputs: the first call's may now be .grad
-        prep = ctx.prepared or _prepare_backward(ctx, *saved[1:], ctx.densification_info, ctx.rasterizer_settings)
-        ctx.prepared = None
-        device = image.device
-        grad_image = grad_image.contiguous()
-        if grad_image.shape != image.shape or grad_image.dtype != torch.float32 or grad_image.device != device:
-            raise ValueError('efgs: the image gradient must be a float32 tensor of the image\'s shape on its device')
-        with _on_device(device):
-            check(lib.efgs_backward(_rasterizer.handle, ctypes.byref(prep.prims), ctypes.byref(prep.settings), ctypes.byref(ctx.frame),
-                                    image.data_ptr(), grad_image.data_ptr(), ctypes.byref(prep.grads), prep.alloc.fn, prep.alloc.ctx,
-                                    _stream(device)))
-            prep.alloc.done()
-        g_means, g_scales, g_rotations, g_opacities, g_pre, g_base, g_res, g_mlp = prep.outputs
-        return (g_means, g_scales, g_rotations, g_opacities,
-                g_pre if g_pre.numel() > 0 else None,
-                g_base if g_base.numel() > 0 else None,
-                g_res if g_res.numel() > 0 else None,
-                g_mlp if g_mlp.numel() > 0 else None,
-                None, None)
-
-
-class _PreparedBackward(NamedTuple):
-    settings: Any       # _lib.Settings
-    keep: list          # tensors the settings point to
-    prims: Any          # _lib.Primitives
-    grads: Any          # _lib.Gradients, pointing into `outputs`
-    outputs: tuple      # gradient tensors, views of one allocation
-    alloc: Any          # _lib.WorkspaceAllocator of the backward
-
-
-def _on_device(device: torch.device):
-    """torch.cuda.device(device) unless it is already current (entering the context costs host time)."""
-    return contextlib.nullcontext() if torch.cuda.current_device() == device.index else torch.cuda.device(device)
-
-
-def _prepare_backward(ctx, means, scales, rotations, opacities, precomputed_colors, base_colors, residual_params, mlp_weights_f32,
-                      dinfo, settings) -> _PreparedBackward:
-    """Native structs, gradient outputs (every gradient is a view of one allocation, each fully written by the
-    backward) and the workspace of the backward of this forward."""
-    device = means.device
-    n = means.shape[0]
-    rows = int(dinfo.shape[0]) if dinfo is not None and dinfo.numel() > 0 else 0
-    if rows and (dinfo.dtype != torch.float32 or not dinfo.is_contiguous() or dinfo.shape[-1] != n or dinfo.device != device):
-        raise ValueError('efgs: densification_info must be a contiguous float32 (2|3, N) tensor on the rendering device')
-    with _on_device(device):
-        cs, keep = _native_settings(settings, device)
-        prims = _native_primitives(means, scales, rotations, opacities, precomputed_colors, base_colors, residual_params, mlp_weights_f32)
-        shapes = [means.shape, scales.shape, rotations.shape, opacities.shape, precomputed_colors.shape, base_colors.shape,
-                  residual_params.shape, (ctx.mlp_numel,)]
-        sizes = [int(torch.Size(sh).numel()) for sh in shapes]
-        flat = torch.empty(sum(sizes), dtype=torch.float32, device=device)
-        outputs = tuple(t.view(sh) for t, sh in zip(flat.split(sizes), shapes))
-        g_means, g_scales, g_rotations, g_opacities, g_pre, g_base, g_res, g_mlp = outputs
-        grads = _lib.Gradients()
-        grads.means, grads.scales, grads.rotations, grads.opacities = (g_means.data_ptr(), g_scales.data_ptr(), g_rotations.data_ptr(),
-                                                                       g_opacities.data_ptr())
-        grads.precomputed_colors = _ptr(g_pre)
-        grads.base_colors = _ptr(g_base)
-        grads.residual_params = _ptr(g_res)
-        grads.mlp_weights = _ptr(g_mlp)
-        grads.densification_info = dinfo.data_ptr() if rows else None
-        grads.densification_rows = rows
-        alloc = _lib.WorkspaceAllocator(device, 'backward')
-    return _PreparedBackward(cs, keep, prims, grads, outputs, alloc)
-
-
 def _empty(device: torch.device, dtype=torch.float32) -> torch.Tensor:
     return torch.empty(0, dtype=dtype, device=device)
 
@@ -304,13 +204,14 @@ def diff_rasterize(means: torch.Tensor, scales: torch.Tensor, rotations: torch.T
                    precomputed_colors: torch.Tensor | None = None, base_colors: torch.Tensor | None = None,
                    residual_params: torch.Tensor | None = None, mlp_weights: torch.Tensor | None = None) -> torch.Tensor:
     """Differentiable render (3, H, W); densification_info (0,) or (2|3, N) is updated in place by the backward."""
-    d = means.device
-    return _Rasterize.apply(means, scales, rotations, opacities,
-                            precomputed_colors if precomputed_colors is not None else _empty(d),
-                            base_colors if base_colors is not None else _empty(d),
-                            residual_params if residual_params is not None else _empty(d),
-                            mlp_weights if mlp_weights is not None else _empty(d),
-                            densification_info, rasterizer_settings)
+    s = rasterizer_settings
+    image, (n, visible, instances, tiles) = _native.diff_rasterize(
+        _rasterizer.handle.value, means, scales, rotations, opacities, densification_info, s.w2c, s.cam_position, s.bg_color,
+        int(s.appearance_degree), int(s.width), int(s.height), float(s.focal_x), float(s.focal_y), float(s.center_x), float(s.center_y),
+        float(s.near_plane), float(s.far_plane), bool(s.proper_antialiasing), bool(s.render_base), bool(s.render_residual),
+        precomputed_colors, base_colors, residual_params, mlp_weights)
+    last_frame_counts.update(n_primitives=n, n_visible=visible, n_instances=instances, n_tiles=tiles)
+    return image
 
 
 @torch.no_grad()
@@ -339,41 +240,6 @@ def rasterize(means: torch.Tensor, scales: torch.Tensor, rotations: torch.Tensor
     return image
 
 
-class _NeuralDecode(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx: Any, features, dirs, mlp_weights, base, degree: int) -> torch.Tensor:
-        device = features.device
-        mlp_half = mlp_weights.detach().half().contiguous()
-        n = int(dirs.shape[0])
-        out = torch.empty((n, 3), dtype=torch.float32, device=device)
-        with torch.cuda.device(device):
-            check(lib.efgs_neural_decode_forward(_rasterizer.handle, n, _ptr(features), _ptr(base), _ptr(dirs), _ptr(mlp_half), int(degree),
-                                                 _ptr(out), _stream(device)))
-        ctx.degree = int(degree)
-        ctx.mlp_numel = mlp_weights.numel()
-        ctx.save_for_backward(features, dirs, mlp_half, base)
-        return out
-
-    @staticmethod
-    @once_differentiable
-    def backward(ctx: Any, grad_out: torch.Tensor):
-        features, dirs, mlp_half, base = ctx.saved_tensors
-        device = features.device
-        n = int(dirs.shape[0])
-        grad_out = grad_out.contiguous()
-        g_features = torch.empty_like(features)
-        g_dirs = torch.empty_like(dirs)
-        g_base = torch.empty_like(base)
-        g_mlp = torch.empty(ctx.mlp_numel, dtype=torch.float32, device=device)
-        with torch.cuda.device(device):
-            alloc = _lib.WorkspaceAllocator(device, 'decode')
-            check(lib.efgs_neural_decode_backward(_rasterizer.handle, n, _ptr(features), _ptr(base), _ptr(dirs), _ptr(mlp_half), ctx.degree,
-                                                  _ptr(grad_out), _ptr(g_features), _ptr(g_base), _ptr(g_dirs), _ptr(g_mlp), alloc.fn,
-                                                  alloc.ctx, _stream(device)))
-            alloc.done()
-        return (g_features if features.numel() > 0 else None, g_dirs, g_mlp, g_base if base.numel() > 0 else None, None)
-
-
 def neural_decode(features: torch.Tensor, dirs: torch.Tensor, mlp_weights: torch.Tensor, degree: int = 1,
                   base_colors: torch.Tensor | None = None) -> torch.Tensor:
     """Differentiable standalone decode of the configured residual MLP (initialize_residual_mlp): raw outputs
@@ -392,7 +258,7 @@ def neural_decode(features: torch.Tensor, dirs: torch.Tensor, mlp_weights: torch
         raise ValueError('efgs: dirs must be (N, 3)')
     if mlp_weights.numel() != _rasterizer.mlp_param_count():
         raise ValueError(f'efgs: mlp_weights must hold {_rasterizer.mlp_param_count()} parameters, got {mlp_weights.numel()}')
-    return _NeuralDecode.apply(features, dirs, mlp_weights, base, degree)
+    return _native.neural_decode(_rasterizer.handle.value, features, dirs, mlp_weights, base, int(degree))
 
 
 @torch.no_grad()
