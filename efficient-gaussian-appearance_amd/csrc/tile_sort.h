@@ -4,9 +4,8 @@
 //   n <= 64, 128, 256 in registers, K = 1, 2, 4 keys per lane (element x = K lane + i): exchanges at distance
 //                     j < K within a lane, j >= K with the lane at xor distance j / K (128 < n <= 192: a
 //                     128-key and a 64-key network merged by rank);
-//   256 < n <= 512    in the wave's LDS slab;
-//   n > 512           chunks of 512 sorted in the slab and written back to the tile's range, then every key
-//                     placed at (its index in its chunk) + (its rank in each other chunk).
+//   n > 256           chunks of 256 sorted by the register network; two of them (n <= 512) merged by rank in the
+//                     wave's LDS slab, more by merge passes through the tile's bucket range in global memory.
 #pragma once
 
 #include "internal.h"
@@ -196,71 +195,98 @@ __device__ __forceinline__ void sort_small_run(const uint4* run, uint32_t n, con
 }
 
 constexpr uint32_t wave_slab = 512;  // keys of a wave's LDS slab
+constexpr uint32_t sort_chunk = 256;  // keys sorted by one register network
 
-// ascending bitonic sort of m (a power of two, <= wave_slab) keys in the wave's slab
-__device__ inline void wave_bitonic_lds(uint64_t* s, uint32_t m, uint32_t lane) {
-    for (uint32_t size = 2; size <= m; size <<= 1) {
-        for (uint32_t j = size >> 1; j > 0; j >>= 1) {
-            for (uint32_t x = lane; x < m; x += 64) {
-                const uint32_t y = x ^ j;
-                if (y > x) {
-                    const uint64_t a = s[x], b = s[y];
-                    if ((a > b) == ((x & size) == 0)) {
-                        s[x] = b;
-                        s[y] = a;
-                    }
-                }
-            }
-            wave_lds_fence();
-        }
-    }
-}
-
-// number of keys below x in the ascending run of bucket entries [0, n)
-__device__ __forceinline__ uint32_t rank_in_bucket(const uint4* run, uint32_t n, uint64_t x) {
-    uint32_t lo = 0, hi = n;
+// The number of keys that `a` (na keys) contributes to the first `diagonal` keys of the merge of the ascending runs a
+// and b (nb keys): keys are unique.
+__device__ __forceinline__ uint32_t merge_split(const uint64_t* a, uint32_t na, const uint64_t* b, uint32_t nb, uint32_t diagonal) {
+    uint32_t lo = diagonal > nb ? diagonal - nb : 0u, hi = min(diagonal, na);
     while (lo < hi) {
         const uint32_t mid = (lo + hi) >> 1;
-        if (key_of(run[mid]) < x) lo = mid + 1; else hi = mid;
+        if (a[mid] < b[diagonal - 1u - mid]) lo = mid + 1; else hi = mid;
     }
     return lo;
 }
 
 // One run of n > forward_sort_max keys (the wave's slab s: wave_slab keys); the sorted arrays in global memory only.
+// Up to 512 keys: both chunks in the slab, a key's position its index in its chunk plus its rank in the other (the
+// 512-key network in the slab that this replaced ran 45 steps of dependent LDS round trips). More: the chunks' keys
+// replace the bucket entries (8 of their 16 bytes each: chunk c's keys end before the entries of chunk c + 1), and
+// merge passes double the sorted length, each lane merging n / 64 consecutive outputs of a pass, between the lower and
+// the upper half of the tile's bucket range (a rank search of every key in every other chunk replaced by log2 passes).
+// Bound by the latency of one wave's dependent steps: 300k Gaussians at 800 x 533 (370 instances per tile on average),
+// forward blend 158 -> 83 us.
 template <typename KeyT>
 __device__ inline void sort_big_run(uint4* bucket, uint2 r, uint32_t n, uint32_t tile, uint32_t* sorted_inst, KeyT* sorted_keys,
                              const uint32_t* inst_prim, uint32_t* sorted_prim, uint32_t lane, uint64_t* s) {
-    uint4* run = bucket + r.x;
+    constexpr uint32_t K = sort_chunk / 64;
+    const uint4* const run = bucket + r.x;
     const SortedOut<KeyT> o{sorted_inst + r.x, sorted_prim + r.x, sorted_keys + r.x, inst_prim, tile, nullptr};
-    if (n <= wave_slab) {
-        uint32_t m = 512;
-        while (m < n) m <<= 1;
-        for (uint32_t x = lane; x < m; x += 64) s[x] = x < n ? key_of(run[x]) : ~0ull;
-        wave_lds_fence();
-        wave_bitonic_lds(s, m, lane);
-        for (uint32_t x = lane; x < n; x += 64) o.put(x, s[x]);
+    const bool in_slab = n <= wave_slab;  // (wave-uniform)
+    uint64_t* const keys = reinterpret_cast<uint64_t*>(bucket + r.x);
+    for (uint32_t c0 = 0; c0 < n; c0 += sort_chunk) {
+        uint64_t k[K];
+        uint32_t l = lane;
+        asm volatile("" : "+v"(l));  // (the network's lane masks are formed per chunk, not kept in registers across them)
+#pragma unroll
+        for (uint32_t i = 0; i < K; i++) {
+            const uint32_t x = c0 + K * l + i;
+            k[i] = x < n ? key_of(run[x]) : ~0ull;
+        }
+        wave_bitonic<K>(k, l);
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // (the chunk's entries are read before its keys overwrite them)
+#pragma unroll
+        for (uint32_t i = 0; i < K; i++) {
+            const uint32_t x = c0 + K * l + i;
+            if (x < n) {
+                if (in_slab) s[x] = k[i];
+                else keys[x] = k[i];
+            }
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // the wave reads the chunks that its lanes wrote
+    if (in_slab) {
+        for (uint32_t x = lane; x < n; x += 64) {
+            const uint64_t key = s[x];
+            const bool first = x < sort_chunk;
+            const uint32_t other = first ? rank_in(s + sort_chunk, n - sort_chunk, key) : rank_in(s, sort_chunk, key);
+            o.put(first ? x + other : x - sort_chunk + other, key);
+        }
         return;
     }
-    const uint32_t n_chunks = (n + wave_slab - 1) / wave_slab;
-    for (uint32_t c = 0; c < n_chunks; c++) {
-        const uint32_t c0 = c * wave_slab, cn = min(wave_slab, n - c0);
-        for (uint32_t x = lane; x < wave_slab; x += 64) s[x] = x < cn ? key_of(run[c0 + x]) : ~0ull;
-        wave_lds_fence();
-        wave_bitonic_lds(s, wave_slab, lane);
-        for (uint32_t x = lane; x < cn; x += 64) run[c0 + x] = make_uint4(static_cast<uint32_t>(s[x]), static_cast<uint32_t>(s[x] >> 32), 0u, 0u);
-        wave_lds_fence();
-    }
-    __threadfence();  // the wave reads back the chunks it wrote
-    for (uint32_t idx = lane; idx < n; idx += 64) {
-        const uint64_t key = key_of(run[idx]);
-        const uint32_t c = idx / wave_slab;
-        uint32_t pos = idx - c * wave_slab;
-        for (uint32_t oc = 0; oc < n_chunks; oc++) {
-            if (oc == c) continue;
-            const uint32_t o0 = oc * wave_slab;
-            pos += rank_in_bucket(run + o0, min(wave_slab, n - o0), key);
+    // (one base pointer and 32-bit positions: n is far below 2^30, a run's range of 2 n keys fits)
+    uint32_t src = 0, dst = n;
+    const uint32_t per = (n + 63u) / 64u;
+    for (uint32_t width = sort_chunk; width < n; width *= 2) {
+        const bool last = 2 * width >= n;
+        uint32_t x = min(lane * per, n);
+        const uint32_t x_end = min(x + per, n);
+        while (x < x_end) {  // the lane's outputs, pair of runs by pair of runs
+            const uint32_t p0 = x & ~(2 * width - 1u), p1 = min(p0 + 2 * width, n);  // (widths are powers of two)
+            const uint32_t na = min(width, n - p0);
+            uint32_t ia = src + p0, ib = ia + na;  // next keys of the two runs
+            const uint32_t ea = ib, eb = src + p1;
+            const uint32_t split = merge_split(keys + ia, na, keys + ib, eb - ib, x - p0);
+            ia += split;
+            ib += x - p0 - split;
+            uint64_t ka = ia < ea ? keys[ia] : ~0ull, kb = ib < eb ? keys[ib] : ~0ull;
+            for (const uint32_t end = min(x_end, p1); x < end; x++) {
+                const bool from_a = ka < kb;  // (a run past its end yields the largest key, which no instance has)
+                const uint64_t key = from_a ? ka : kb;
+                if (from_a) {
+                    ia++;
+                    ka = ia < ea ? keys[ia] : ~0ull;
+                } else {
+                    ib++;
+                    kb = ib < eb ? keys[ib] : ~0ull;
+                }
+                if (last) o.put(x, key);
+                else keys[dst + x] = key;
+            }
         }
-        o.put(pos, key);
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+        src = n - src;
+        dst = n - dst;
     }
 }
 
