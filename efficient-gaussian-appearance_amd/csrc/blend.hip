@@ -277,8 +277,8 @@ __device__ __forceinline__ uint32_t row_min_u32(uint32_t v) {
 // pixel per lane, that this replaced: 14 % fewer VALU instructions and a third of the LDS reads per pixel, at the
 // same time, 70.6 against 70.5 us on the 1M-Gaussian 1080p scene: both waited on the gather chain emission index
 // -> primitive -> record; with the primitives read from the sorted array it takes 57 us.)
-template <typename KeyT>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(7))) void blend_forward_kernel(BlendForwardArgs a) {
+template <typename KeyT, bool SEGMENTS>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(SEGMENTS ? 6 : 7))) void blend_forward_kernel(BlendForwardArgs a) {
     if (a.overflow && *a.overflow != 0) return;  // the binning was skipped: the host re-runs the frame
     constexpr uint32_t CHUNK = 32;
     constexpr uint32_t RING = 2 * CHUNK;
@@ -387,6 +387,19 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(7))) void bl
         if (__builtin_amdgcn_ballot_w64(T[0] >= transmittance_threshold || T[1] >= transmittance_threshold ||
                                         T[2] >= transmittance_threshold) == 0)
             break;
+        // a segment of the backward starts here: no group has walked into this chunk yet (the window was closed)
+        uint64_t closed = 0;  // the next chunk's hits while the window ends at this chunk
+        if (SEGMENTS) {
+            if (base > 0 && base % a.segment == 0) {
+                float4* const out = a.checkpoints + static_cast<size_t>(range.x / a.segment + base / a.segment) * tile_pixels;
+#pragma unroll
+                for (uint32_t r = 0; r < 3; r++) out[(ly0 + r) * tile_width + lx] = make_float4(T[r], cr[r], cg[r], cb[r]);
+            }
+            if ((base + CHUNK) % a.segment == 0) {
+                closed = M & 0xffffffff00000000ull;
+                M ^= closed;
+            }
+        }
         const uint32_t half = c & 1u, flip = half * CHUNK;  // (wave-uniform) ring index of window position j: j ^ flip
         const PrimRecord rec_n = a.records[p_next];          // chunk c + 2
         p_next = load_p(base + 3 * CHUNK);                   // chunk c + 3
@@ -460,6 +473,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(7))) void bl
             wave_lds_fence();
             m2 = cull(half, min(CHUNK, n_total - nb));
         }
+        if (SEGMENTS) M |= closed;
         M = (M >> 32) | (static_cast<uint64_t>(m2) << 32);
     }
 
@@ -492,7 +506,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(7))) void bl
     if (lane == 0) a.tile_max[tile] = wm;
 }
 
-template <bool ABS, uint32_t LIST>
+template <bool ABS, uint32_t LIST, bool SEGMENTS>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(EFGS_BACKWARD_WAVES))) void blend_backward_kernel(BlendBackwardArgs a) {
     constexpr uint32_t CHUNK = backward_chunk;
     constexpr uint32_t NX = ABS ? 3u : 1u;                 // values after the first eight (w g_b; |dL/dmean2d|)
@@ -521,7 +535,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(EFGS_BACKWAR
     const float pxf = static_cast<float>(px) + 0.5f;
     const uint2 range = a.ranges[tile];
     const uint32_t n_total = range.y - range.x;
-    const uint32_t n_proc = min(n_total, a.tile_max[tile]);
+    const uint32_t n_walk = min(n_total, a.tile_max[tile]);  // instances up to the tile's last contributor
+    // this wave's instances: the whole list, or (SEGMENTS) segment blockIdx.y of it; the last wave of a tile goes on to
+    // the list's end
+    const uint32_t n_begin = SEGMENTS ? blockIdx.y * a.segment : 0u;
+    const uint32_t n_proc = SEGMENTS && blockIdx.y + 1 < gridDim.y ? min(n_walk, n_begin + a.segment) : n_walk;
+    if (SEGMENTS && blockIdx.y > 0 && n_begin >= n_walk) return;
     if (lane < VS) s_part[zero_rec * VS + lane] = 0.0f;
     if (lane < 3) s_stage[0][lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 
@@ -563,6 +582,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(EFGS_BACKWAR
             const float gbg = Tf[r] * -(gr[r] * bg0 + gg[r] * bg1 + gb[r] * bg2);
             Ab[r] = inside[r] ? A - gbg : 0.0f;
         }
+        if (SEGMENTS && n_begin > 0) {  // the forward's state at the segment's start: T, and the colour so far leaves Ab
+            const float4* const in = a.checkpoints + static_cast<size_t>(range.x / a.segment + blockIdx.y) * tile_pixels;
+            float4 ck[3];
+#pragma unroll
+            for (uint32_t r = 0; r < 3; r++) ck[r] = in[(ly0 + r) * tile_width + lx];
+#pragma unroll
+            for (uint32_t r = 0; r < 3; r++) {
+                T[r] = inside[r] ? ck[r].x : 1.0f;
+                Ab[r] -= __builtin_fmaf(ck[r].w, gb[r], __builtin_fmaf(ck[r].z, gg[r], ck[r].y * gr[r]));
+            }
+        }
     }
 
     // where the lane stores its sums: value 4m + {0, 2, 1, 3}[k] of group i (m = 0, 1; the extras: 8 + the same),
@@ -593,14 +623,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(EFGS_BACKWAR
     // the next chunk's top), and no loaded value is copied between loop-carried registers (a copy would make the
     // loop wait for the load).
     uint32_t p_next = 0;  // primitive indices of chunk b + 1
-    if (n_proc > 0) {
-        const uint32_t e0 = load_e(0), p0 = load_p(0);
-        p_next = load_p(CHUNK);
+    if (n_proc > n_begin) {
+        const uint32_t e0 = load_e(n_begin), p0 = load_p(n_begin);
+        p_next = load_p(n_begin + CHUNK);
         const PrimRecord rec0 = a.records[p0];
-        stage(0, rec0, e0);
+        stage(n_begin, rec0, e0);
     }
     const uint32_t gx0 = bx0 + 4u * (i & 3u), gy0 = by0 + ly0;  // the lane's group rectangle: 4 x 3 pixels
-    for (uint32_t base = 0; base < n_proc; base += CHUNK) {
+    for (uint32_t base = n_begin; base < n_proc; base += CHUNK) {
         // advance the gather pipeline: records and emission indices of chunk b + 1, primitive indices of b + 2
         const PrimRecord rec_n = a.records[p_next];
         const uint32_t e_n = load_e(base + CHUNK);
@@ -824,7 +854,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(EFGS_BACKWAR
         if (base + CHUNK < n_proc) stage(base + CHUNK, rec_n, e_n);  // the next chunk
     }
     // instances the tile never reached (after every pixel's last contributor) get zero records
-    for (uint32_t q = n_proc + lane; q < n_total; q += 64) {
+    if (SEGMENTS && blockIdx.y > 0) return;
+    for (uint32_t q = n_walk + lane; q < n_total; q += 64) {
         const uint32_t e = a.sorted_inst[range.x + q];
         float* const out = a.inst_grads + RECORD * static_cast<uint64_t>(e);
         const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -983,10 +1014,12 @@ __global__ __launch_bounds__(256) void accumulate_scores_kernel(const uint32_t* 
 
 bool launch_blend_forward(const BlendForwardArgs& a, hipStream_t s) {
     if (a.n_tiles == 0) return true;
-    if (a.key_bytes == 2)
-        blend_forward_kernel<uint16_t><<<a.n_tiles, 64, 0, s>>>(a);
+    if (a.segment > 0)  // (few tiles: 16-bit tile keys)
+        blend_forward_kernel<uint16_t, true><<<a.n_tiles, 64, 0, s>>>(a);
+    else if (a.key_bytes == 2)
+        blend_forward_kernel<uint16_t, false><<<a.n_tiles, 64, 0, s>>>(a);
     else
-        blend_forward_kernel<uint32_t><<<a.n_tiles, 64, 0, s>>>(a);
+        blend_forward_kernel<uint32_t, false><<<a.n_tiles, 64, 0, s>>>(a);
     EFGS_HIP_CHECK(hipGetLastError());
     return true;
 }
@@ -1004,12 +1037,33 @@ bool launch_pruning_scores(const BlendBackwardArgs& a, const uint32_t* n_touched
     return true;
 }
 
+// Segments only where the tiles alone leave most of the GPU's wave slots (four backward waves on each of 1,024 SIMDs)
+// empty: about 8,192 per frame at two instances per primitive, of at least one 32-instance chunk (4,096 and 16,384
+// measured 106 and 101 us for 102 us in the 300k frame below, the forward 88 and 93 us for 90 us). Measured, backward and
+// forward (which records the states and closes its window at a segment's end): 256 tiles of 100 instances 43 -> 18 and
+// 24 -> 26 us; 2,250 tiles of 370 (300k Gaussians at 800 x 533) 133 -> 102 and 83 -> 90 us; 3,350 tiles of 96 64 -> 59
+// and 32 -> 37 us; 5,382 tiles of 97 101 -> 105 and 45 -> 47 us: the line lies at 3,072 tiles. The rule reads nothing
+// that changes between frames of a scene (the instance capacity does), so gradients stay reproducible bit for bit.
+uint32_t instances_per_segment(uint64_t n_primitives, uint32_t n_tiles) {
+    constexpr uint64_t wanted = 8192;
+    if (n_tiles == 0 || n_tiles >= 3072) return 0;
+    const uint64_t chunks = 2 * n_primitives / (wanted * backward_chunk) + 1;
+    return static_cast<uint32_t>(chunks) * backward_chunk;
+}
+
 bool launch_blend_backward(const BlendBackwardArgs& a, hipStream_t s) {
     if (a.n_tiles == 0) return true;
-    if (a.abs_grads)
-        blend_backward_kernel<true, backward_list_abs><<<a.n_tiles, 64, 0, s>>>(a);
-    else
-        blend_backward_kernel<false, backward_list><<<a.n_tiles, 64, 0, s>>>(a);
+    const dim3 grid(a.n_tiles, a.segment > 0 ? a.n_segment_blocks : 1u);
+    if (a.segment > 0) {
+        if (a.abs_grads)
+            blend_backward_kernel<true, backward_list_abs, true><<<grid, 64, 0, s>>>(a);
+        else
+            blend_backward_kernel<false, backward_list, true><<<grid, 64, 0, s>>>(a);
+    } else if (a.abs_grads) {
+        blend_backward_kernel<true, backward_list_abs, false><<<grid, 64, 0, s>>>(a);
+    } else {
+        blend_backward_kernel<false, backward_list, false><<<grid, 64, 0, s>>>(a);
+    }
     EFGS_HIP_CHECK(hipGetLastError());
     return true;
 }

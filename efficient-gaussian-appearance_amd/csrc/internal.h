@@ -139,7 +139,13 @@ struct BlendForwardArgs {
     uint32_t width, height, grid_w, n_tiles;
     uint32_t hwc;                  // image layout (H, W, 3)
     uint32_t clamp;                // image clamped to [0, 1] (NaN to 0)
+    float4* checkpoints;           // (slots x 192) per segment start: T and colour of every pixel (null: no segments)
+    uint32_t segment;              // instances per segment, a multiple of 32 (0: no segments)
 };
+// Small frames: the backward walks a tile's list in segments, one wave each, from the transmittance and colour that the
+// forward recorded at the segment's start (0: whole lists). Segment k >= 1 of the tile whose instances start at s has
+// the slot s / segment + k: the slots of a frame's segments are distinct and at most (instances) / segment.
+uint32_t instances_per_segment(uint64_t n_primitives, uint32_t n_tiles);
 bool launch_blend_forward(const BlendForwardArgs& a, hipStream_t s);
 
 struct BlendBackwardArgs {
@@ -157,6 +163,9 @@ struct BlendBackwardArgs {
     float* inst_grads;             // (I x 9, or I x 12 with abs_grads), emission order (pruning scores: one float per instance)
     uint32_t width, height, grid_w, n_tiles;
     uint32_t abs_grads;            // also reduce |dL/dmean2d| (third densification row)
+    const float4* checkpoints;     // the forward's, with its segment length (segment 0: whole lists)
+    uint32_t segment;
+    uint32_t n_segment_blocks;     // blocks per tile; the last one walks every segment from its own on
 };
 bool launch_blend_backward(const BlendBackwardArgs& a, hipStream_t s);
 // pruning scores of the frame in `a` (grad_image unused): per-instance scores into a.inst_grads, then
