@@ -334,9 +334,13 @@ uint32_t mlp_weight_bytes(const MlpShape& m) {
     return (halves * 2 + 15) / 16 * 16;
 }
 
-// the forward's neural kernels (preprocess, decode): weights + 4 per-wave staging areas of 64 rows of
-// (n_in_padded + 4) halves
-uint32_t mlp_smem_forward(const MlpShape& m) { return mlp_weight_bytes(m) + 4 * 64 * (m.n_in_padded + 4) * 2; }
+// the forward's neural kernels (preprocess, decode): the weights W_l (rows padded by 8 halves, no transposes) + 4
+// per-wave staging areas of 64 rows of (n_in_padded + 4) halves
+uint32_t mlp_smem_forward(const MlpShape& m) {
+    uint32_t halves = 0;
+    for (uint32_t l = 0; l <= m.n_hidden; l++) halves += (l == m.n_hidden ? 16u : m.n_neurons) * ((l == 0 ? m.n_in_padded : m.n_neurons) + 8);
+    return (halves * 2 + 15) / 16 * 16 + 4 * 64 * (m.n_in_padded + 4) * 2;
+}
 
 constexpr uint32_t max_dynamic_lds = 160 * 1024;  // gfx950: 160 KiB of LDS per block
 

@@ -30,8 +30,8 @@ extern "C" __global__ __launch_bounds__(256, 2) void EFGS_KERNEL_NAME(efgs::Neur
     const uint32_t wave = threadIdx.x >> 6;
     extern __shared__ __align__(16) unsigned char smem[];
     const _Float16* WL = reinterpret_cast<const _Float16*>(smem);
-    _Float16* stage = reinterpret_cast<_Float16*>(smem + nn::WEIGHT_BYTES) + wave * 64 * nn::XS;
-    nn::load_weights<decode_block>(a.mlp_weights, reinterpret_cast<uint16_t*>(smem), threadIdx.x);
+    _Float16* stage = reinterpret_cast<_Float16*>(smem + nn::FORWARD_WEIGHT_BYTES) + wave * 64 * nn::XS;
+    nn::load_weights<decode_block, false>(a.mlp_weights, reinterpret_cast<uint16_t*>(smem), threadIdx.x);
     __syncthreads();
     const uint32_t n_chunks = (a.n + decode_block - 1) / decode_block;
     // the lane's raw inputs (features, base colour, direction) of its primitive in the block's next chunk, loaded
@@ -84,7 +84,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void EFGS_CAT(EFGS_KERNEL_NAME, 
     extern __shared__ __align__(16) unsigned char smem[];
     const _Float16* WL = reinterpret_cast<const _Float16*>(smem);
     _Float16* stage = reinterpret_cast<_Float16*>(smem + nn::WEIGHT_BYTES + wave * nn::STAGE_BYTES);
-    nn::load_weights<decode_block>(a.mlp_weights, reinterpret_cast<uint16_t*>(smem), threadIdx.x);
+    nn::load_weights<decode_block, true>(a.mlp_weights, reinterpret_cast<uint16_t*>(smem), threadIdx.x);
 
     nn::f4 dW[nn::NL][nn::NT][nn::KT];
 #pragma unroll

@@ -189,8 +189,8 @@ extern "C" __global__ __launch_bounds__(256, 4) void EFGS_KERNEL_NAME(efgs::Prep
     // residual MLP weights staged once per block (padded rows); staging rows of the MLP inputs (64 per wave)
     extern __shared__ __align__(16) unsigned char smem[];
     const _Float16* WL = reinterpret_cast<const _Float16*>(smem);
-    _Float16* stage = reinterpret_cast<_Float16*>(smem + nn::WEIGHT_BYTES);
-    nn::load_weights<preprocess_block>(a.mlp_weights, reinterpret_cast<uint16_t*>(smem), threadIdx.x);
+    _Float16* stage = reinterpret_cast<_Float16*>(smem + nn::FORWARD_WEIGHT_BYTES);
+    nn::load_weights<preprocess_block, false>(a.mlp_weights, reinterpret_cast<uint16_t*>(smem), threadIdx.x);
     __syncthreads();
 #endif
     const uint32_t n_chunks = (a.n + preprocess_block - 1) / preprocess_block;
