@@ -34,16 +34,16 @@ constexpr float min_alpha = 1.0f / 255.0f;
 //   r0 = (mean2d.x, mean2d.y, conic.x, conic.y)
 //   r1 = (conic.z, opacity, color.r, color.g)
 //   r2 = (color.b, bits(x_min | x_max << 16), bits(y_min | y_max << 16), bits(first-tiles mask))
-// where bit j of the mask (j < 4) records whether tile j of the primitive's tile rectangle (row-major order)
+// where bit j of the mask (j < n_sequential_tiles) records whether tile j of the primitive's tile rectangle (row-major order)
 // passes the contribution test, as the preprocess counted it, so instance emission need not test those again
 struct PrimRecord {
     float4 r0, r1, r2;
 };
 
-// tiles of a primitive's rectangle that the preprocess tests one per lane (and records in the first-tiles mask);
-// further tiles are tested wave-cooperatively, by the preprocess and again by instance emission. Eight rather than
-// four: a wave's cooperative loop takes one primitive per step, however few tiles it has past the first ones
-// (100k SH3 Gaussians at 800x800: emission 37.5 -> 21.4 us, preprocess 24.6 -> 21.4 us; neutral on 1M at 1080p)
+// tiles of a primitive's rectangle whose test results the preprocess records in the first-tiles mask; instance
+// emission takes these one per lane and tests the further tiles again, wave-cooperatively. Eight rather than
+// four: the cooperative loop takes one primitive per step, however few tiles it has past the first ones
+// (emission of 100k SH3 Gaussians at 800x800: 37.5 -> 21.4 us; neutral on 1M at 1080p)
 constexpr uint32_t n_sequential_tiles = 8;
 static_assert(n_sequential_tiles <= 32, "the first-tiles mask is one 32-bit word of the record");
 // floats per instance gradient record of the blend backward (dL/dmean2d 2, dL/dconic 3, dL/dopacity, dL/dcolour 3;
