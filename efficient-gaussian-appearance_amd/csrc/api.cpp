@@ -187,6 +187,7 @@ struct PrimitiveLayout {
     uint32_t* n_touched;
     uint32_t* depth_keys;
     PrimRecord* records;
+    uint2* tile_rects;
     uint32_t* prim_offset;
     uint32_t* block_counts;
     uint32_t* block_key_ranges;
@@ -203,6 +204,7 @@ struct PrimitiveLayout {
         l.n_touched = c.take<uint32_t>(nn);
         l.depth_keys = c.take<uint32_t>(nn);
         l.records = c.take<PrimRecord>(nn);
+        l.tile_rects = c.take<uint2>(nn);
         l.prim_offset = c.take<uint32_t>(nn);
         l.block_counts = c.take<uint32_t>(2ull * blocks);
         l.block_key_ranges = c.take<uint32_t>(2ull * blocks);
@@ -731,6 +733,7 @@ int forward_impl(efgs_rasterizer* r, const efgs_primitives* prims, const efgs_se
         a.n_touched = pl.n_touched;
         a.depth_keys = pl.depth_keys;
         a.records = pl.records;
+        a.tile_rects = pl.tile_rects;
         a.block_counts = pl.block_counts;
         a.block_key_ranges = pl.block_key_ranges;
         a.counters = pl.counters;
@@ -780,6 +783,7 @@ int forward_impl(efgs_rasterizer* r, const efgs_primitives* prims, const efgs_se
         ca.prim_offset_out = pl.prim_offset;
         ca.n_touched = pl.n_touched;
         ca.records = pl.records;
+        ca.tile_rects = pl.tile_rects;
         ca.keys = il.keys;
         ca.inst_prim = il.inst_prim;
         ca.counters = pl.counters;

@@ -59,7 +59,8 @@ struct CreateInstancesArgs {
     uint32_t* visible_prims_out;   // the fused path writes the compaction (the same arrays)
     uint32_t* prim_offset_out;
     uint32_t* n_touched;
-    const PrimRecord* records;
+    const PrimRecord* records;     // read for large rectangles only
+    const uint2* tile_rects;
     void* keys;                // tile key per emission slot, key_bytes wide
     uint32_t* inst_prim;
     uint32_t* counters;        // the visible count is read here ([0]); nothing is emitted when [counter_overflow] is set

@@ -4,8 +4,9 @@
 // index), without a global sort:
 //   create_instances    (fused, grids whose tile histogram fits the LDS) blocks of contiguous primitives scan
 //                       the preprocess's tile counts (the compaction: visible primitives in index order and
-//                       their first emission slots) and emit (tile key, primitive) at the emission slots, the
-//                       tile test of the preprocess for every tile past its recorded first ones; each block
+//                       their first emission slots) and emit (tile key, primitive) at the emission slots, from
+//                       the tile mask that the preprocess recorded (rectangles of more tiles than the mask has
+//                       bits are tested again); each block
 //                       counts its instances per tile in an LDS histogram (ranks from the atomics' return
 //                       values) and writes its row of the segment x tile table. Larger grids: compact_visible,
 //                       then one thread per visible primitive, counted per tile with global atomics;
@@ -62,7 +63,6 @@ __device__ __forceinline__ uint32_t wave_reduce(uint32_t v, OP op) {
 __device__ __forceinline__ uint32_t wave_sum(uint32_t v) { return wave_reduce(v, [](uint32_t x, uint32_t y) { return x + y; }); }
 // a lane's value in every lane; the lane index must be wave-uniform
 __device__ __forceinline__ uint32_t lane_value(uint32_t v, uint32_t src) { return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(src))); }
-__device__ __forceinline__ float lane_value(float v, uint32_t src) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), static_cast<int>(src))); }
 
 __global__ __launch_bounds__(preprocess_block) void compact_visible_kernel(const uint32_t* n_touched, const uint32_t* block_offsets,
                                                                           uint32_t* visible_out, uint32_t* prim_offset, uint32_t n) {
@@ -89,101 +89,117 @@ __global__ __launch_bounds__(preprocess_block) void compact_visible_kernel(const
     prim_offset[p] = off + inc - touched;
 }
 
-// Emission of one visible primitive per thread (visible index i, index order): (tile key, primitive) for every
-// tile of its tile rectangle that passes the contribution test, the first 8 tiles per lane from the test results
-// the preprocess recorded in the primitive's record, larger footprints' further tiles tested again
-// wave-cooperatively (64 tiles per step, positions from ballot prefix counts); emit(slot, tile) is
-// called by the lane that writes each instance. Emission slots are [prim_offset, prim_offset + n_touched); a
-// count that disagrees with the preprocess is clamped to that range, the remainder padded with an out-of-range
-// key (never bucketed) and counted in counters[2]. A primitive that emitted fewer tiles than counted gets
-// n_touched lowered to the emitted count, so the per-primitive sums of the backward and of the pruning scores
-// cover only slots that a blend kernel writes. Every lane of the wave must call this (ballots and shuffles).
-// The fields of a primitive's 48-byte record that emission reads (nine of its twelve words: not the colour).
-struct EmitRecord {
-    float4 r0;               // mean2d x, y, conic x, y
-    float cz, opacity;       // conic z, opacity
-    uint32_t bx, by, first;  // packed screen bounds x, y; the first-tiles mask
-};
-__device__ __forceinline__ EmitRecord load_emit_record(const PrimRecord* records, uint32_t p) {
-    const float* const r = reinterpret_cast<const float*>(records + p);
-    const float4 r0 = *reinterpret_cast<const float4*>(r);
-    const float2 r1 = *reinterpret_cast<const float2*>(r + 4);
-    return EmitRecord{r0, r1.x, r1.y, __float_as_uint(r[9]), __float_as_uint(r[10]), __float_as_uint(r[11])};
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-
-// n: the primitive's tile count from the preprocess, rec: its record's emission fields (both loaded by the caller).
-template <typename KeyT, typename Emit>
-__device__ __forceinline__ void emit_primitive_rec(const CreateInstancesArgs& a, uint32_t p, uint32_t off, uint32_t n, const EmitRecord& rec, bool active,
-                                                   uint32_t lane, Emit&& emit) {
-    const uint64_t lanes_below = (1ull << lane) - 1ull;
-    const uint32_t bx = rec.bx, by = rec.by;
-    const TileRect t = screen_to_tile_bounds(bx & 0xffffu, bx >> 16, by & 0xffffu, by >> 16);
-    const uint32_t bw = t.x1 - t.x0;
-    const uint32_t cnt = active ? bw * (t.y1 - t.y0) : 0u;
-    const float smx = rec.r0.x - 0.5f, smy = rec.r0.y - 0.5f;
-    const float cx = rec.r0.z, cy = rec.r0.w, cz = rec.cz;
-    const float pt = cnt > n_sequential_tiles ? power_threshold_of(rec.opacity) : 0.0f;  // (the tile test of the later tiles)
-    const uint32_t first_tiles = rec.first;  // the preprocess's test of the first n_sequential_tiles tiles
-    KeyT* keys = static_cast<KeyT*>(a.keys);
-    uint32_t k = 0;
-    for (uint32_t j = 0; j < cnt && j < n_sequential_tiles; j++) {
-        const uint32_t tx = t.x0 + j % bw, ty = t.y0 + j / bw;
-        if ((first_tiles >> j) & 1u) {
-            if (k < n) {
-                const uint32_t tile = ty * a.grid_w + tx;
-                keys[off + k] = static_cast<KeyT>(tile);
-                a.inst_prim[off + k] = p;
-                emit(off + k, tile);
-            }
-            k++;
+__device__ __forceinline__ uint32_t wave_inclusive_max(uint32_t v) {
+    v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x111, 0xf, 0xf, true)));
+    v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x112, 0xf, 0xf, true)));
+    v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x114, 0xf, 0xf, true)));
+    v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x118, 0xf, 0xf, true)));
+    v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x142, 0xa, 0xf, false)));
+    v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x143, 0xc, 0xf, false)));
+    return v;
+}
+// another lane's value (the lane index may differ between lanes; the source lane must be active)
+__device__ __forceinline__ uint32_t from_lane(uint32_t v, uint32_t src) {
+    return static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(static_cast<int>(src * 4u), static_cast<int>(v)));
+}
+// index of the k-th set bit (k from 0, less than the number of set bits)
+__device__ __forceinline__ uint32_t nth_set_bit(uint32_t m, uint32_t k) {
+    uint32_t pos = 0;
+#pragma unroll
+    for (uint32_t half = 16; half > 0; half >>= 1) {
+        const uint32_t c = static_cast<uint32_t>(__popc((m >> pos) & ((1u << half) - 1u)));
+        if (k >= c) {
+            k -= c;
+            pos += half;
         }
     }
-    uint64_t coop = __ballot(cnt > n_sequential_tiles);
+    return pos;
+}
+
+// Emission of a wave's primitives, one per lane (n: the tile count from the preprocess, 0 for none; off: the first
+// emission slot; rect: its tile rectangle and mask, see pack_tile_rect; primitive_of(lane): a lane's primitive):
+// (tile key, primitive) for every tile that the primitive reaches, its tiles in row-major order. emit(slot, tile) is
+// called by the lane that writes each instance. Every lane of the wave must call this (lane exchanges); marks: 64
+// words of LDS of the wave's own.
+//
+// The wave's instances are laid end to end, the primitives in lane order, and written 64 at a time, one per lane: the
+// stores of a step are contiguous, and a wave takes as many steps as its instances fill, where a loop over each
+// lane's own tiles takes as many as the largest primitive has (plus one per primitive past the loop's bound), and reads
+// 12 bytes per primitive in place of most of its 48-byte record: 10k Gaussians at 256 x 192 10.4 -> 7.1 us, 100k at
+// 800 x 800 12.8 -> 8.4, 300k at 800 x 533 20.0 -> 11.9, 1M at 1080p 28.3 -> 20.3 (the preprocess's 8 bytes more per
+// primitive: + 2). Only a
+// rectangle of more than mask_tiles tiles is tested again, from its record, by the whole wave, 64 tiles per step,
+// positions from ballot prefix counts. Its emission slots are [off, off + n); a count that disagrees with the
+// preprocess is clamped to that range, the remainder padded with an out-of-range key (never bucketed) and counted in
+// counters[2], and n_touched lowered to the emitted count, so that the per-primitive sums of the backward and of the
+// pruning scores cover only slots that a blend kernel writes.
+template <typename KeyT, typename Prim, typename Emit>
+__device__ __forceinline__ void emit_wave(const CreateInstancesArgs& a, uint32_t off, uint32_t n, uint2 rect, uint32_t lane, uint32_t* marks,
+                                          Prim&& primitive_of, Emit&& emit) {
+    KeyT* keys = static_cast<KeyT*>(a.keys);
+    const bool large = n > 0 && rect.x >> 26 == large_rect;
+    const uint32_t small = large ? 0u : n;
+    const uint32_t end = wave_inclusive_sum(small), start = end - small;
+    const uint32_t total = lane_value(end, 63);
+    for (uint32_t w0 = 0; w0 < total; w0 += 64) {
+        // the owner of every instance of the window: the last lane whose instances start at or before it
+        marks[lane] = 0u;
+        if (small > 0 && start < w0 + 64u && end > w0) marks[max(start, w0) - w0] = lane + 1u;
+        wave_lds_sync();
+        const uint32_t owner = max(wave_inclusive_max(marks[lane]), 1u) - 1u;
+        wave_lds_sync();  // the marks are read before the next window's
+        const uint32_t xyw = from_lane(rect.x, owner), mask = from_lane(rect.y, owner);
+        const uint32_t k = w0 + lane - from_lane(start, owner), slot = from_lane(off, owner) + k;
+        const uint32_t p = primitive_of(owner);
+        if (w0 + lane < total) {
+            const uint32_t j = nth_set_bit(mask, k), bw = xyw >> 26;
+            const uint32_t dy = static_cast<uint32_t>((static_cast<float>(j) + 0.5f) * __builtin_amdgcn_rcpf(static_cast<float>(bw)));  // j / bw (j < 32)
+            const uint32_t tile = ((xyw >> 13 & 0x1fffu) + dy) * a.grid_w + (xyw & 0x1fffu) + j - dy * bw;
+            keys[slot] = static_cast<KeyT>(tile);
+            a.inst_prim[slot] = p;
+            emit(slot, tile);
+        }
+    }
+    const uint64_t lanes_below = (1ull << lane) - 1ull;
+    uint64_t coop = __ballot(large);
     while (coop != 0) {
         const uint32_t src = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(__ffsll(static_cast<long long>(coop)) - 1));
         coop &= coop - 1;
-        const uint32_t c_x0 = lane_value(t.x0, src), c_y0 = lane_value(t.y0, src), c_bw = lane_value(bw, src), c_cnt = lane_value(cnt, src);
-        const uint32_t c_off = lane_value(off, src), c_n = lane_value(n, src), c_p = lane_value(p, src);
-        const float c_mx = lane_value(smx, src), c_my = lane_value(smy, src);
-        const float c_cx = lane_value(cx, src), c_cy = lane_value(cy, src), c_cz = lane_value(cz, src), c_pt = lane_value(pt, src);
-        uint32_t c_k = lane_value(k, src);
-        for (uint32_t base = n_sequential_tiles; base < c_cnt; base += 64) {
+        const uint32_t c_off = lane_value(off, src), c_n = lane_value(n, src), c_p = __builtin_amdgcn_readfirstlane(primitive_of(src));
+        const PrimRecord rec = a.records[c_p];
+        const uint32_t bx = __float_as_uint(rec.r2.y), by = __float_as_uint(rec.r2.z);
+        const TileRect t = screen_to_tile_bounds(bx & 0xffffu, bx >> 16, by & 0xffffu, by >> 16);
+        const uint32_t bw = t.x1 - t.x0, cnt = bw * (t.y1 - t.y0);
+        const float pt = power_threshold_of(rec.r1.y);
+        uint32_t k = 0;
+        for (uint32_t base = 0; base < cnt; base += 64) {
             const uint32_t j = base + lane;
-            const uint32_t tx = c_x0 + j % c_bw, ty = c_y0 + j / c_bw;
-            const bool hit = j < c_cnt && will_primitive_contribute(c_mx, c_my, c_cx, c_cy, c_cz, tx, ty, c_pt);
+            const uint32_t tx = t.x0 + j % bw, ty = t.y0 + j / bw;
+            const bool hit = j < cnt && will_primitive_contribute(rec.r0.x - 0.5f, rec.r0.y - 0.5f, rec.r0.z, rec.r0.w, rec.r1.x, tx, ty, pt);
             const uint64_t m = __ballot(hit);
-            const uint32_t pos = c_k + static_cast<uint32_t>(__popcll(m & lanes_below));
+            const uint32_t pos = k + static_cast<uint32_t>(__popcll(m & lanes_below));
             if (hit && pos < c_n) {
                 const uint32_t tile = ty * a.grid_w + tx;
                 keys[c_off + pos] = static_cast<KeyT>(tile);
                 a.inst_prim[c_off + pos] = c_p;
                 emit(c_off + pos, tile);
             }
-            c_k += static_cast<uint32_t>(__popcll(m));
+            k += static_cast<uint32_t>(__popcll(m));
         }
-        if (lane == src) k = c_k;
-    }
-    if (active && k != n) {
-        for (uint32_t j = (k < n ? k : n); j < n; j++) {
-            keys[off + j] = static_cast<KeyT>(~static_cast<KeyT>(0));
-            a.inst_prim[off + j] = p;
+        if (lane == src && k != c_n) {
+            for (uint32_t j = min(k, c_n); j < c_n; j++) {
+                keys[c_off + j] = static_cast<KeyT>(~static_cast<KeyT>(0));
+                a.inst_prim[c_off + j] = c_p;
+            }
+            if (k < c_n) a.n_touched[c_p] = k;
+            atomicAdd(&a.counters[2], 1u);
         }
-        if (k < n) a.n_touched[p] = k;
-        atomicAdd(&a.counters[2], 1u);
     }
-}
-
-template <typename KeyT, typename Emit>
-__device__ __forceinline__ void emit_primitive_at(const CreateInstancesArgs& a, uint32_t p, uint32_t off, bool active, uint32_t lane, Emit&& emit) {
-    emit_primitive_rec<KeyT>(a, p, off, a.n_touched[p], load_emit_record(a.records, p), active, lane, emit);
-}
-
-// visible primitive i (index order) of the compacted list; inactive lanes repeat the last one
-template <typename KeyT, typename Emit>
-__device__ __forceinline__ void emit_primitive(const CreateInstancesArgs& a, uint32_t i_raw, bool active, uint32_t lane, Emit&& emit) {
-    const uint32_t i = active ? i_raw : a.n_visible - 1;
-    const uint32_t p = a.visible_prims[i];
-    emit_primitive_at<KeyT>(a, p, a.prim_offset[p], active, lane, emit);
 }
 
 // One thread per visible primitive (the path for grids whose tile histogram does not fit the LDS).
@@ -192,8 +208,11 @@ __global__ __launch_bounds__(instance_block) void create_instances_kernel(Create
     if (a.counters[counter_overflow] != 0) return;
     a.n_visible = a.counters[0];
     if (blockIdx.x * instance_block >= a.n_visible) return;  // (block-uniform: the grid covers a bound on V)
-    const uint32_t i = blockIdx.x * instance_block + threadIdx.x;
-    emit_primitive<KeyT>(a, i, i < a.n_visible, threadIdx.x & 63u, [](uint32_t, uint32_t) {});
+    __shared__ uint32_t s_marks[instance_block];
+    const uint32_t i = blockIdx.x * instance_block + threadIdx.x, lane = threadIdx.x & 63u;
+    const uint32_t p = a.visible_prims[min(i, a.n_visible - 1u)];  // (threads past the list: the last one, with no instances)
+    emit_wave<KeyT>(a, a.prim_offset[p], i < a.n_visible ? a.n_touched[p] : 0u, a.tile_rects[p], lane, s_marks + (threadIdx.x - lane),
+                    [&](uint32_t owner) { return from_lane(p, owner); }, [](uint32_t, uint32_t) {});
 }
 
 // Emission with the per-tile counts, the compaction and the counter scan in one kernel (grids whose histogram
@@ -204,33 +223,34 @@ __global__ __launch_bounds__(instance_block) void create_instances_kernel(Create
 // chunks before its own (its first visible index and emission slot). More instances than the buffers hold set the
 // overflow flag and nothing is emitted. Then, 1024 primitives at a time (a round), a block scan of the visible
 // flags and tile counts gives every visible primitive its visible index and first emission slot (visible_prims,
-// prim_offset: the compaction), and the thread that holds the primitive emits it, counted per tile in an LDS
+// prim_offset: the compaction), and the wave that holds the primitives emits them, counted per tile in an LDS
 // histogram whose atomic return values rank every instance among the segment's instances of its tile (in arbitrary
 // order: the per-tile sort fixes the order later); it stores rank | s << 24 per instance and writes its histogram
-// row table[s][*]. The tile counts and records of the first two rounds are loaded
+// row table[s][*]. The tile counts and rectangles of the first two rounds are loaded
 // before the chunk counts are summed and every later round's during the round two before it, so the rounds wait on
-// no global load of their own (a thread whose primitive is not visible loads a record it does not use).
+// no global load of their own (a thread whose primitive is not visible loads a rectangle it does not use).
 constexpr uint32_t fused_block = 1024;
 template <typename KeyT>
 __global__ __launch_bounds__(fused_block) void create_instances_fused_kernel(CreateInstancesArgs a, FusedBinningArgs f, uint32_t* local_rank,
                                                                            uint32_t* table, uint32_t n_tiles) {
     extern __shared__ uint32_t hist[];  // n_tiles counters
     __shared__ uint32_t s_red[fused_block / 64][8];
+    __shared__ uint32_t s_marks[fused_block];
     __shared__ uint32_t s_scan[2][fused_block / 64][2];  // the rounds' wave totals, alternating between rounds
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t seg = blockIdx.x;
     const uint32_t c0 = seg * f.chunks_per_segment, c1 = min(f.n_chunks, c0 + f.chunks_per_segment);
     const uint32_t p_begin = c0 * preprocess_block, p_end = min(f.n_prims, c1 * preprocess_block);  // (p_end > p_begin)
-    // the tile counts and records of a round (threads past the segment: count 0, the segment's last record)
-    const auto load_round = [&](uint32_t it, uint32_t& touched, EmitRecord& rec) {
+    // the tile counts and rectangles of a round (threads past the segment: count 0, the segment's last rectangle)
+    const auto load_round = [&](uint32_t it, uint32_t& touched, uint2& rect) {
         const uint32_t p = p_begin + it * fused_block + tid;
         touched = p < p_end ? a.n_touched[p] : 0u;
-        rec = load_emit_record(a.records, min(p, p_end - 1u));
+        rect = a.tile_rects[min(p, p_end - 1u)];
     };
     uint32_t touched_a, touched_b;
-    EmitRecord rec_a, rec_b;
-    load_round(0, touched_a, rec_a);
-    load_round(1, touched_b, rec_b);
+    uint2 rect_a, rect_b;
+    load_round(0, touched_a, rect_a);
+    load_round(1, touched_b, rect_b);
 
     // totals, depth-key range and the segment's prefix from the per-chunk counts
     uint32_t tv = 0, ti = 0, bv = 0, bi = 0, kmin = 0xffffffffu, kmax = 0u;
@@ -283,7 +303,7 @@ __global__ __launch_bounds__(fused_block) void create_instances_fused_kernel(Cre
     uint32_t run_v = bv, run_i = bi;
     // A round's scan partials alternate between two buffers: a wave writes round r + 2's partials only after the
     // barrier of round r + 1, which every wave reaches after its reads of round r's.
-    const auto round = [&](uint32_t it, uint32_t touched, const EmitRecord& rec) {
+    const auto round = [&](uint32_t it, uint32_t touched, uint2 rect) {
         const uint32_t p = p_begin + it * fused_block + tid;
         const uint32_t vis = touched > 0 ? 1u : 0u;
         const uint32_t iv = wave_inclusive_sum(vis), ii = wave_inclusive_sum(touched);  // inclusive wave scans
@@ -307,9 +327,8 @@ __global__ __launch_bounds__(fused_block) void create_instances_fused_kernel(Cre
             a.visible_prims_out[run_v + vpos] = p;
             a.prim_offset_out[p] = off;
         }
-        emit_primitive_rec<KeyT>(a, p, off, touched, rec, vis != 0u, lane, [&](uint32_t slot, uint32_t tile) {
-            local_rank[slot] = tag | atomicAdd(&hist[tile], 1u);
-        });
+        emit_wave<KeyT>(a, off, touched, rect, lane, s_marks + (tid - lane), [&](uint32_t owner) { return p - lane + owner; },
+                        [&](uint32_t slot, uint32_t tile) { local_rank[slot] = tag | atomicAdd(&hist[tile], 1u); });
         run_v += nv;
         run_i += ni;
     };
@@ -317,11 +336,11 @@ __global__ __launch_bounds__(fused_block) void create_instances_fused_kernel(Cre
     // registers: a copy would wait for the load)
     const uint32_t n_rounds = (p_end - p_begin + fused_block - 1u) / fused_block;
     for (uint32_t it = 0; it < n_rounds; it += 2) {  // (block-uniform)
-        round(it, touched_a, rec_a);
-        if (it + 2 < n_rounds) load_round(it + 2, touched_a, rec_a);
+        round(it, touched_a, rect_a);
+        if (it + 2 < n_rounds) load_round(it + 2, touched_a, rect_a);
         if (it + 1 >= n_rounds) break;
-        round(it + 1, touched_b, rec_b);
-        if (it + 3 < n_rounds) load_round(it + 3, touched_b, rec_b);
+        round(it + 1, touched_b, rect_b);
+        if (it + 3 < n_rounds) load_round(it + 3, touched_b, rect_b);
     }
     __syncthreads();
     uint32_t* row = table + static_cast<size_t>(seg) * n_tiles;

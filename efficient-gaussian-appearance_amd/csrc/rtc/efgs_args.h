@@ -35,6 +35,7 @@ struct PreprocessForwardArgs {
     uint32_t* n_touched;          // (N) 0 for culled primitives
     uint32_t* depth_keys;         // (N) float bits of the view depth
     PrimRecord* records;          // (N) written for visible primitives
+    uint2* tile_rects;            // (N) written for visible primitives: pack_tile_rect, mask of the tiles it reaches
     uint32_t* block_counts;       // (2 * blocks) visible count and instance count per block
     uint32_t* block_key_ranges;   // (2 * blocks) min and max depth key of the block's visible primitives
     uint32_t* counters;           // the frame's counters: [2] (instance-emission mismatches) is cleared here

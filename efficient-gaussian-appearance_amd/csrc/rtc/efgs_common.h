@@ -35,17 +35,24 @@ constexpr float min_alpha = 1.0f / 255.0f;
 //   r1 = (conic.z, opacity, color.r, color.g)
 //   r2 = (color.b, bits(x_min | x_max << 16), bits(y_min | y_max << 16), bits(first-tiles mask))
 // where bit j of the mask (j < n_sequential_tiles) records whether tile j of the primitive's tile rectangle (row-major order)
-// passes the contribution test, as the preprocess counted it, so instance emission need not test those again
+// passes the contribution test, as the preprocess counted it
 struct PrimRecord {
     float4 r0, r1, r2;
 };
 
-// tiles of a primitive's rectangle whose test results the preprocess records in the first-tiles mask; instance
-// emission takes these one per lane and tests the further tiles again, wave-cooperatively. Eight rather than
-// four: the cooperative loop takes one primitive per step, however few tiles it has past the first ones
-// (emission of 100k SH3 Gaussians at 800x800: 37.5 -> 21.4 us; neutral on 1M at 1080p)
+// tiles of a primitive's rectangle whose test results the record's spare word holds
 constexpr uint32_t n_sequential_tiles = 8;
 static_assert(n_sequential_tiles <= 32, "the first-tiles mask is one 32-bit word of the record");
+// What instance emission reads of a visible primitive (8 bytes, beside its tile count): its tile rectangle's first
+// tile and width in one word, and bit j of the second word for tile j of the rectangle (row-major) if the primitive
+// reaches it. A rectangle of more than mask_tiles tiles has the width large_rect: emission reads its record and tests
+// its tiles again.
+constexpr uint32_t mask_tiles = 32;
+constexpr uint32_t large_rect = 63;
+__device__ __forceinline__ uint32_t pack_tile_rect(uint32_t x0, uint32_t y0, uint32_t width) {  // (images of at most 65535 x 65535)
+    return x0 | y0 << 13 | width << 26;
+}
+static_assert(65536 / tile_width <= 1 << 13 && 65536 / tile_height <= 1 << 13, "a tile coordinate fits 13 bits");
 // floats per instance gradient record of the blend backward (dL/dmean2d 2, dL/dconic 3, dL/dopacity, dL/dcolour 3;
 // with |dL/dmean2d| for three densification rows: 2 more and a pad)
 constexpr uint32_t record_floats = 9;

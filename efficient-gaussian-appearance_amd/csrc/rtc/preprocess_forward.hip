@@ -133,7 +133,7 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v, OP op) {
 }
 
 // exact number of tiles in the tile rectangle that the primitive reaches; first_tiles receives the test results of
-// the rectangle's first n_sequential_tiles tiles (bit i: tile i, row-major). Every lane of the wave must call it.
+// the rectangle's first mask_tiles tiles (bit i: tile i, row-major). Every lane of the wave must call it.
 // The wave's (primitive, tile) pairs are laid end to end, the primitives in lane order, and tested 64 at a time, one
 // per lane: as many tests as the wave's rectangles hold tiles, where a loop over each lane's own rectangle takes as
 // many steps as the largest of the 64 (and needs a second, cooperative loop for the large ones). With the colour
@@ -180,11 +180,10 @@ __device__ inline uint32_t count_touched_tiles(const Projected& pr, uint32_t lan
             const uint32_t n = hi - lo;  // 1..64
             const uint64_t own = (m >> lo) & (~0ull >> (64u - n));
             touched += static_cast<uint32_t>(__popcll(own));
-            if (w0 + lo - start < n_sequential_tiles) first_tiles |= static_cast<uint32_t>(own) << (w0 + lo - start);
+            if (w0 + lo - start < mask_tiles) first_tiles |= static_cast<uint32_t>(own) << (w0 + lo - start);
         }
         wave_lds_sync();  // the marks are read before the next window's
     }
-    first_tiles &= (1u << n_sequential_tiles) - 1u;
     return touched;
 }
 
@@ -291,6 +290,10 @@ extern "C" __global__ __launch_bounds__(256, 4) void EFGS_KERNEL_NAME(efgs::Prep
             a.n_touched[p] = touched;
             a.depth_keys[p] = key;
         }
+        if (visible) {
+            const uint32_t bw = pr.tiles.x1 - pr.tiles.x0, cnt = bw * (pr.tiles.y1 - pr.tiles.y0);
+            a.tile_rects[p] = make_uint2(pack_tile_rect(pr.tiles.x0, pr.tiles.y0, cnt <= mask_tiles ? bw : large_rect), first_tiles);
+        }
         // whether a block barrier follows the last read of wave_counts in this chunk (else one ends the chunk)
         bool counts_released = false;
 
@@ -393,7 +396,7 @@ extern "C" __global__ __launch_bounds__(256, 4) void EFGS_KERNEL_NAME(efgs::Prep
             rec.r0 = make_float4(pr.mean2d_x, pr.mean2d_y, pr.conic_x, pr.conic_y);
             rec.r1 = make_float4(pr.conic_z, pr.opacity, color.x, color.y);
             rec.r2 = make_float4(color.z, __uint_as_float(pr.sx0 | (pr.sx1 << 16)), __uint_as_float(pr.sy0 | (pr.sy1 << 16)),
-                                 __uint_as_float(first_tiles));
+                                 __uint_as_float(first_tiles & ((1u << n_sequential_tiles) - 1u)));
             a.records[p] = rec;
         }
         // (block-uniform) wave_counts, or the MLP's output rows, read before the next chunk writes them

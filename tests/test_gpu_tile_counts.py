@@ -1,4 +1,5 @@
-"""The preprocess's tile tests (csrc/rtc/preprocess_forward.hip, count_touched_tiles): waves whose rectangles fill less than
+"""The preprocess's tile tests (csrc/rtc/preprocess_forward.hip, count_touched_tiles) and the emission from their masks
+(csrc/raster.hip, emit_wave; the last two frames: the largest grid that the fused kernel takes, and one past it): waves whose rectangles fill less than
 one window of 64 tests, straddle windows, or hold more than 2^15 tile-width products (a division per test instead of the
 reciprocal product), with last waves that are partly or wholly invisible. Counts, first-tiles masks and the emitted
 instances exactly equal the oracle's."""
@@ -13,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize('model', ['precomputed', 'sh', 'neural'])
 @pytest.mark.parametrize('n,width,height,shift', [(1, 16, 12, 0.0), (63, 64, 48, 0.0), (64, 130, 77, 1.0), (65, 130, 77, 3.0), (257, 333, 222, 2.0),
-                                                  (700, 1600, 1200, 3.0), (130, 3000, 2400, 5.0)])
+                                                  (700, 1600, 1200, 3.0), (130, 3000, 2400, 5.0),
+                                                  (2000, 2048, 1536, 2.0), (1500, 4160, 3180, 2.0)])
 def test_tile_counts(model, n, width, height, shift):
     import torch
     from efgs.rasterization import forward_with_frame, frame_views
