@@ -799,11 +799,11 @@ int forward_impl(efgs_rasterizer* r, const efgs_primitives* prims, const efgs_se
         t.end(s);
         t.begin(EFGS_STAGE_TILE_BUCKETS, s);
         if (!launch_tile_buckets(plan, il.keys, key_bytes, il.inst_prim, pl.depth_keys, il.table, il.local_rank, ts, il.bucket, max_instances,
-                                 n_tiles, s))
+                                 tl.ranges, n_tiles, s))
             return EFGS_ERR_HIP;
         t.end(s);
         t.begin(EFGS_STAGE_TILE_SORT, s);
-        if (!launch_tile_ranges(ts, tl.ranges, n_tiles, s)) return EFGS_ERR_HIP;
+        if (!launch_tile_ranges(ts, tl.ranges, max_instances, n_tiles, s)) return EFGS_ERR_HIP;
         t.end(s);
 
         BlendForwardArgs b;

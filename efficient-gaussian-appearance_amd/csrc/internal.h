@@ -92,7 +92,7 @@ bool launch_create_instances(const CreateInstancesArgs& a, int key_bytes, const 
 // instance count, descending (longest-processing-time-first list scheduling, so that a kernel's last blocks are
 // short ones). The count is bucketed into 64 classes (1 + 4 floor(log2 n) + the next two bits, reversed; an empty
 // tile is the last class); the column scan counts each 64-tile block's tiles per class and gives every tile its
-// rank among them (lane order), one small kernel turns the counts into each (block, class) run's first position,
+// rank among them (lane order), the bucket kernel's first blocks turn the counts into each (block, class) run's first position,
 // and the tile sort writes every tile at its position. Deterministic; a tile's result does not depend on it.
 constexpr uint32_t order_classes = 64;
 struct TileScan {
@@ -111,18 +111,20 @@ struct TileScan {
 bool launch_tile_counts(const TileBinning& plan, const void* keys, int key_bytes, uint32_t max_instances, uint32_t* table, const TileScan& ts,
                         uint32_t n_tiles, hipStream_t s);
 // every instance's bucket entry (emission index, depth key of its primitive, primitive, 0; the low 8 bytes are the
-// sort key depth key << 32 | emission index) into a slot of its tile's range
+// sort key depth key << 32 | emission index) into a slot of its tile's range; on grids of up to 16,384 tiles also
+// every tile's range and place in the blends' tile order (see launch_tile_ranges)
 bool launch_tile_buckets(const TileBinning& plan, const void* keys, int key_bytes, const uint32_t* inst_prim, const uint32_t* depth_keys,
                          const uint32_t* table, const uint32_t* local_rank, const TileScan& ts, uint4* bucket, uint32_t max_instances,
-                         uint32_t n_tiles, hipStream_t s);
-// per tile: [start, end) into ranges and its place in the blends' tile order (the runs are sorted by the forward blend)
-bool launch_tile_ranges(const TileScan& ts, uint2* ranges, uint32_t n_tiles, hipStream_t s);
+                         uint2* ranges, uint32_t n_tiles, hipStream_t s);
+// per tile: [start, end) into ranges and its place in the blends' tile order (the runs are sorted by the forward blend);
+// nothing where launch_tile_buckets has written them
+bool launch_tile_ranges(const TileScan& ts, uint2* ranges, uint32_t max_instances, uint32_t n_tiles, hipStream_t s);
 bool launch_reduce_partials(const float* partials, uint32_t n_blocks, uint32_t n_params, float* out, hipStream_t s);
 
 struct BlendForwardArgs {
     const uint2* ranges;
     uint4* bucket;                 // per tile slot: emission index, depth key, primitive, 0 (unsorted; runs of more
-                                   // than 512 are sorted in chunks in place)
+                                   // than 512 are sorted and merged in place)
     uint32_t* sorted_inst;         // emission index per sorted instance (written here)
     uint32_t* sorted_prim;         // primitive per sorted instance (written here)
     void* sorted_keys;             // tile key per sorted instance (key_bytes wide; written here)
