@@ -816,7 +816,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(EFGS_BACKWAR
 // one step, which it stores in the group's slot row of the Gaussian's ring entry. When every group has left a chunk,
 // two lanes per Gaussian add its sixteen slots in a fixed order into one float at the instance's emission slot
 // (instances after every pixel's last contributor get 0). No atomics (the reference adds per pixel with float atomics).
-// 400k SH3 Gaussians at 1080p: 56 us, against 64 us for three waves of eight 4x2 groups, one pixel per lane, whose
+// 400k SH3 Gaussians at 1296 x 840: 56 us, against 64 us for three waves of eight 4x2 groups, one pixel per lane, whose
 // batches waited at block barriers and read every Gaussian from LDS for one pixel per lane.
 // Reference: B/rasterization/include/kernels_pruning_scores.cuh:11-171.
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void blend_scores_kernel(BlendBackwardArgs a) {

@@ -138,7 +138,7 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v, OP op) {
 // per lane: as many tests as the wave's rectangles hold tiles, where a loop over each lane's own rectangle takes as
 // many steps as the largest of the 64 (and needs a second, cooperative loop for the large ones). With the colour
 // read beside the projection's inputs, against eight tiles per lane and a cooperative step per larger primitive:
-// 10k SH3 Gaussians at 256 x 192 14.1 -> 11.3 us, 150k SV at 1237 x 823 26.9 -> 21.1, 400k SH3 at 1080p 35.9 -> 32.8,
+// 10k SH3 Gaussians at 256 x 192 14.1 -> 11.3 us, 150k SV at 1237 x 823 26.9 -> 21.1, 400k SH3 at 1296 x 840 35.9 -> 32.8,
 // 1M neural at 1080p 57.3 -> 51.5.
 __device__ inline uint32_t count_touched_tiles(const Projected& pr, uint32_t lane, unsigned char* area, uint32_t& first_tiles) {
 #pragma clang fp contract(off)
