@@ -16,6 +16,7 @@ constexpr float lobe_eps_norm = 1e-8f;
 constexpr float lobe_cos_limit = 0.999999f;
 constexpr float lobe_sin_limit = 1.41421321e-3f;  // sqrt(1 - lobe_cos_limit^2)
 constexpr float lobe_pole_limit = 0.99999988f;
+constexpr float lobe_min_om = 2.38418579e-7f;  // 1 - lobe_pole_limit^2
 constexpr float lobe_shape_limit = 1e4f;
 constexpr float lobe_freq_scale = 20.0f;
 constexpr float lobe_log2e = 1.44269504088896340736f, lobe_ln2 = 0.69314718055994530942f;
@@ -24,8 +25,9 @@ constexpr float lobe_log2e = 1.44269504088896340736f, lobe_ln2 = 0.6931471805599
 // lobe kernels issued 6.6e7 (forward) and 1.16e8 (backward) VALU instructions for 8 lobes on 1M Gaussians, most of them
 // in the library's tanh, exp and log and in correctly rounded divides and square roots; 4.0e7 and 7.6e7 now (NASG
 // backward 213 -> 181 us at 1080p, the training step 581 -> 555 us; the forward then waits on its row reads). The
-// results are as close to 64 bits as before: an angle's sine comes as sech x instead of sqrt(1 - tanh^2 x), which
-// cancelled.
+// results are as close to 64 bits as before or closer: an angle's sine comes as sech x instead of sqrt(1 - tanh^2 x),
+// which cancelled, and the backward takes 1 - vz^2 and, near the antipole, K without cancellation (a lobe seen at
+// vz = -1 + 3.3e-7 had its frame gradients off by a quarter to nine tenths before).
 
 // tanh x and sech x = sqrt(1 - tanh^2 x) from u = exp(-|x|): (1 - u^2) / (1 + u^2) with the sign of x, 2 u / (1 + u^2)
 __device__ __forceinline__ float lobe_tanh(float x, float& sech) {
@@ -137,8 +139,13 @@ __device__ inline float3 lobe_residual_backward(const float* p, float3 gc, float
         const float w2 = residual_activation<RES_ACT>(p[wo + 2]);
         const float vz = lobe_dot(d, f.z), vx = lobe_dot(d, f.x);
         const float vzc = clampf(vz, -lobe_pole_limit, lobe_pole_limit);
-        const float K = __builtin_fmaf(0.5f, vzc, 0.5f);
-        const float rom = __builtin_amdgcn_rcpf(__builtin_fmaf(-vzc, vzc, 1.0f));
+        // 1 - vz^2 as the sum of the other components' squares, and K = (1 + vz) / 2 towards the antipole from it: both
+        // differences cancel near vz = -1, where the gradient of log K holds their quotient
+        const float cs = f.cp * f.su;
+        const float vy = d.z * (f.sp * f.su) + d.y * (f.ct * f.cu - f.st * cs) - d.x * (f.ct * cs + f.st * f.cu);
+        const float om = fmaxf(vx * vx + vy * vy, lobe_min_om);
+        const float rom = __builtin_amdgcn_rcpf(om);
+        const float K = vzc < 0.0f ? 0.5f * om * __builtin_amdgcn_rcpf(1.0f - vzc) : __builtin_fmaf(0.5f, vzc, 0.5f);
         const float vx2 = vx * vx, avr = an * vx * rom;
         const float Ke = __builtin_fmaf(an * vx2, rom, lobe_eps);
         const float logK2 = __builtin_amdgcn_logf(K);
