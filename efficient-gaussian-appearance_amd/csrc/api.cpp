@@ -258,10 +258,10 @@ struct InstanceLayout {
     uint32_t* sorted_inst;   // emission slots in (tile, depth, primitive) order
     void* sorted_keys;       // tile key of every sorted instance
     uint32_t* sorted_prim;   // primitive of every sorted instance
-    float4* checkpoints;     // per segment start: T and colour of the tile's pixels (small frames' backward)
+    float4* checkpoints;     // per segment start: T and colour of the tile's pixels (frames of few tiles with a backward; else null)
     size_t bytes;
 
-    static InstanceLayout carve(char* base, uint64_t n_instances, int key_bytes, uint32_t n_tiles, uint64_t n_primitives) {
+    static InstanceLayout carve(char* base, uint64_t n_instances, int key_bytes, uint32_t n_tiles, bool segments) {
         InstanceLayout l;
         Carver c{base};
         const uint64_t ni = n_instances > 0 ? n_instances : 1;
@@ -274,8 +274,7 @@ struct InstanceLayout {
         l.sorted_inst = c.take<uint32_t>(ni);
         l.sorted_keys = c.take_bytes(key_bytes * ni);
         l.sorted_prim = c.take<uint32_t>(ni);
-        const uint32_t segment = instances_per_segment(n_primitives, n_tiles);
-        l.checkpoints = c.take<float4>(segment > 0 ? (ni / segment + 1) * tile_pixels : 1);
+        l.checkpoints = segments && n_tiles < segmented_tiles ? c.take<float4>(segment_slots(ni) * tile_pixels) : nullptr;
         l.bytes = c.offset + buffer_alignment;
         return l;
     }
@@ -680,9 +679,10 @@ int wait_counters(efgs_rasterizer* r, uint32_t seq, hipStream_t s) {
 
 // The forward pipeline. A training forward (frame != null) keeps the backward state (final T, last contributors,
 // tile maxima) and writes the image CHW; an inference render (frame == null) writes only the image, in CHW or
-// HWC layout, optionally clamped. segments: record the states that the backward's segments start from.
+// HWC layout, optionally clamped. segments: record the states that the backward's segments start from (frames that get
+// a backward). counts (optional): primitives, visible primitives, instances, tiles.
 int forward_impl(efgs_rasterizer* r, const efgs_primitives* prims, const efgs_settings* settings, float* image, efgs_alloc_fn alloc,
-                 void* alloc_ctx, efgs_frame* frame, bool hwc, bool clamp, bool segments, void* stream) {
+                 void* alloc_ctx, efgs_frame* frame, bool hwc, bool clamp, bool segments, void* stream, int64_t* counts = nullptr) {
     if (!r || !prims || !settings || !image || !alloc) return fail(EFGS_ERR_INVALID_ARGUMENT, "null argument");
     if (settings->width <= 0 || settings->height <= 0 || settings->width > 65535 || settings->height > 65535)
         return fail(EFGS_ERR_INVALID_ARGUMENT, "image size out of range");
@@ -766,7 +766,7 @@ int forward_impl(efgs_rasterizer* r, const efgs_primitives* prims, const efgs_se
     // max_instances: bounds on the counts, the grid sizes).
     InstanceLayout il{};
     const auto bin_and_blend = [&](char* iblob, uint64_t cap, uint32_t max_visible, uint32_t max_instances) -> int {
-        il = InstanceLayout::carve(iblob, cap, key_bytes, n_tiles, n);
+        il = InstanceLayout::carve(iblob, cap, key_bytes, n_tiles, segments);
         FusedBinningArgs fa{};
         const TileBinning plan = fused ? fused_binning_plan(n, n_tiles, fa.chunks_per_segment) : TileBinning{false, 0u, 1u};
         fa.block_counts = pl.block_counts;
@@ -830,7 +830,6 @@ int forward_impl(efgs_rasterizer* r, const efgs_primitives* prims, const efgs_se
         b.hwc = hwc ? 1u : 0u;
         b.clamp = clamp ? 1u : 0u;
         if (!frame) b.final_T = nullptr;
-        b.segment = segments ? instances_per_segment(n, n_tiles) : 0u;
         b.checkpoints = il.checkpoints;
         t.begin(EFGS_STAGE_BLEND_FORWARD, s);
         if (!launch_blend_forward(b, s)) return EFGS_ERR_HIP;
@@ -840,7 +839,7 @@ int forward_impl(efgs_rasterizer* r, const efgs_primitives* prims, const efgs_se
 
     char* iblob = nullptr;
     if (speculate) {
-        iblob = static_cast<char*>(alloc(alloc_ctx, InstanceLayout::carve(nullptr, capacity, key_bytes, n_tiles, n).bytes));
+        iblob = static_cast<char*>(alloc(alloc_ctx, InstanceLayout::carve(nullptr, capacity, key_bytes, n_tiles, segments).bytes));
         if (!iblob) return fail(EFGS_ERR_ALLOC, "allocation of the instance buffers failed");
         if (int c = bin_and_blend(iblob, capacity, n, static_cast<uint32_t>(capacity))) return c;
     }
@@ -862,9 +861,15 @@ int forward_impl(efgs_rasterizer* r, const efgs_primitives* prims, const efgs_se
         // the binning and the blend): exact buffers, with the overflow flag cleared
         if (speculate && !launch_fill_u32(pl.counters + counter_overflow, 0u, 1, s)) return EFGS_ERR_HIP;
         capacity = n_instances;
-        iblob = static_cast<char*>(alloc(alloc_ctx, InstanceLayout::carve(nullptr, capacity, key_bytes, n_tiles, n).bytes));
+        iblob = static_cast<char*>(alloc(alloc_ctx, InstanceLayout::carve(nullptr, capacity, key_bytes, n_tiles, segments).bytes));
         if (!iblob) return fail(EFGS_ERR_ALLOC, "allocation of the instance buffers failed");
         if (int c = bin_and_blend(iblob, capacity, n_visible, n_instances)) return c;
+    }
+    if (counts) {
+        counts[0] = n;
+        counts[1] = n_visible;
+        counts[2] = n_instances;
+        counts[3] = n_tiles;
     }
     if (!frame) return EFGS_OK;
 
@@ -895,6 +900,11 @@ int efgs_render(efgs_rasterizer* r, const efgs_primitives* prims, const efgs_set
     return forward_impl(r, prims, settings, image, alloc, alloc_ctx, nullptr, to_chw == 0, clamp_output != 0, false, stream);
 }
 
+int efgs_forward_no_backward(efgs_rasterizer* r, const efgs_primitives* prims, const efgs_settings* settings, float* image, efgs_alloc_fn alloc,
+                             void* alloc_ctx, int64_t* counts, void* stream) {
+    return forward_impl(r, prims, settings, image, alloc, alloc_ctx, nullptr, false, false, false, stream, counts);
+}
+
 int efgs_backward(efgs_rasterizer* r, const efgs_primitives* prims, const efgs_settings* settings, const efgs_frame* frame, const float* image,
                   const float* grad_image, efgs_gradients* grads, efgs_alloc_fn alloc, void* alloc_ctx, void* stream) {
     if (!r || !prims || !settings || !frame || !image || !grad_image || !grads || !alloc)
@@ -919,7 +929,7 @@ int efgs_backward(efgs_rasterizer* r, const efgs_primitives* prims, const efgs_s
     const uint32_t n_instances = static_cast<uint32_t>(frame->n_instances);
     const PrimitiveLayout pl = PrimitiveLayout::carve(static_cast<char*>(frame->primitive_buffers), n);
     const TileLayout tl = TileLayout::carve(static_cast<char*>(frame->tile_buffers), n_tiles);
-    const InstanceLayout il = InstanceLayout::carve(static_cast<char*>(frame->instance_buffers), instance_capacity(*frame), frame->key_bytes, n_tiles, n);
+    const InstanceLayout il = InstanceLayout::carve(static_cast<char*>(frame->instance_buffers), instance_capacity(*frame), frame->key_bytes, n_tiles, true);
     const uint32_t* sorted_inst = il.sorted_inst;
 
     const size_t grad_bytes = static_cast<size_t>(n_instances > 0 ? n_instances : 1) *
@@ -945,10 +955,10 @@ int efgs_backward(efgs_rasterizer* r, const efgs_primitives* prims, const efgs_s
     b.grid_w = grid_w;
     b.n_tiles = n_tiles;
     b.abs_grads = grads->densification_rows > 2 ? 1u : 0u;
-    b.segment = instances_per_segment(n, n_tiles);
     b.checkpoints = il.checkpoints;
+    b.segment = instances_per_segment(n_instances);
     // twice the average tile's segments and two more (the last wave of a tile walks the rest of its list)
-    b.n_segment_blocks = b.segment > 0 ? 2 * div_up(n_instances, static_cast<uint64_t>(n_tiles) * b.segment) + 2 : 1u;
+    b.n_segment_blocks = 2 * div_up(n_instances, static_cast<uint64_t>(n_tiles) * b.segment) + 2;
     StageTimer& t = r->timer;
     t.begin(EFGS_STAGE_BLEND_BACKWARD, s);
     if (!launch_blend_backward(b, s)) return EFGS_ERR_HIP;
@@ -1065,7 +1075,7 @@ int efgs_update_pruning_scores(efgs_rasterizer* r, const efgs_primitives* prims,
     const uint32_t n_instances = static_cast<uint32_t>(frame.n_instances);
     const PrimitiveLayout pl = PrimitiveLayout::carve(static_cast<char*>(frame.primitive_buffers), n);
     const TileLayout tl = TileLayout::carve(static_cast<char*>(frame.tile_buffers), n_tiles);
-    const InstanceLayout il = InstanceLayout::carve(static_cast<char*>(frame.instance_buffers), instance_capacity(frame), frame.key_bytes, n_tiles, n);
+    const InstanceLayout il = InstanceLayout::carve(static_cast<char*>(frame.instance_buffers), instance_capacity(frame), frame.key_bytes, n_tiles, false);
     float* inst_scores = static_cast<float*>(alloc(alloc_ctx, static_cast<size_t>(n_instances) * sizeof(float)));
     if (!inst_scores) return fail(EFGS_ERR_ALLOC, "allocation of the instance score buffer failed");
     BlendBackwardArgs b;
@@ -1132,7 +1142,7 @@ int efgs_get_frame_views(const efgs_frame* frame, efgs_frame_views* v) {
     const uint32_t n_tiles = static_cast<uint32_t>(frame->grid_width) * static_cast<uint32_t>(frame->grid_height);
     const PrimitiveLayout pl = PrimitiveLayout::carve(static_cast<char*>(frame->primitive_buffers), n);
     const TileLayout tl = TileLayout::carve(static_cast<char*>(frame->tile_buffers), n_tiles);
-    const InstanceLayout il = InstanceLayout::carve(static_cast<char*>(frame->instance_buffers), instance_capacity(*frame), frame->key_bytes, n_tiles, n);
+    const InstanceLayout il = InstanceLayout::carve(static_cast<char*>(frame->instance_buffers), instance_capacity(*frame), frame->key_bytes, n_tiles, false);
     v->n_touched = pl.n_touched;
     v->depth_keys = pl.depth_keys;
     v->records = reinterpret_cast<const float*>(pl.records);

@@ -238,6 +238,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(SEGMENTS ? 6
     const float pxf = static_cast<float>(px) + 0.5f;
     const uint2 range = a.ranges[tile];
     const uint32_t n_total = range.y - range.x;
+    const uint32_t segment = SEGMENTS ? instances_per_segment(a.counters[1]) : 0u;
     // The tile's run is sorted here: the emission indices, primitives and tile keys in (depth, primitive) order for
     // the backward; a run that fits the register networks also leaves its primitives in LDS for the walk, a longer
     // one (LDS slab, chunks) is read back from the sorted array.
@@ -329,12 +330,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(SEGMENTS ? 6
         // a segment of the backward starts here: no group has walked into this chunk yet (the window was closed)
         uint64_t closed = 0;  // the next chunk's hits while the window ends at this chunk
         if (SEGMENTS) {
-            if (base > 0 && base % a.segment == 0) {
-                float4* const out = a.checkpoints + static_cast<size_t>(range.x / a.segment + base / a.segment) * tile_pixels;
+            if (base > 0 && base % segment == 0) {
+                float4* const out = a.checkpoints + static_cast<size_t>(range.x / segment + base / segment) * tile_pixels;
 #pragma unroll
                 for (uint32_t r = 0; r < 3; r++) out[(ly0 + r) * tile_width + lx] = make_float4(T[r], cr[r], cg[r], cb[r]);
             }
-            if ((base + CHUNK) % a.segment == 0) {
+            if ((base + CHUNK) % segment == 0) {
                 closed = M & 0xffffffff00000000ull;
                 M ^= closed;
             }
@@ -987,7 +988,7 @@ __global__ __launch_bounds__(256) void accumulate_scores_kernel(const uint32_t* 
 
 bool launch_blend_forward(const BlendForwardArgs& a, hipStream_t s) {
     if (a.n_tiles == 0) return true;
-    if (a.segment > 0)  // (few tiles: 16-bit tile keys)
+    if (a.checkpoints)  // (few tiles: 16-bit tile keys)
         blend_forward_kernel<uint16_t, true><<<a.n_tiles, 64, 0, s>>>(a);
     else if (a.key_bytes == 2)
         blend_forward_kernel<uint16_t, false><<<a.n_tiles, 64, 0, s>>>(a);
@@ -1010,24 +1011,10 @@ bool launch_pruning_scores(const BlendBackwardArgs& a, const uint32_t* n_touched
     return true;
 }
 
-// Segments only where the tiles alone leave most of the GPU's wave slots (four backward waves on each of 1,024 SIMDs)
-// empty: about 8,192 per frame at two instances per primitive, of at least one 32-instance chunk (4,096 and 16,384
-// measured 106 and 101 us for 102 us in the 300k frame below, the forward 88 and 93 us for 90 us). Measured, backward and
-// forward (which records the states and closes its window at a segment's end): 256 tiles of 100 instances 43 -> 18 and
-// 24 -> 26 us; 2,250 tiles of 370 (300k Gaussians at 800 x 533) 133 -> 102 and 83 -> 90 us; 3,350 tiles of 96 64 -> 59
-// and 32 -> 37 us; 5,382 tiles of 97 101 -> 105 and 45 -> 47 us: the line lies at 3,072 tiles. The rule reads nothing
-// that changes between frames of a scene (the instance capacity does), so gradients stay reproducible bit for bit.
-uint32_t instances_per_segment(uint64_t n_primitives, uint32_t n_tiles) {
-    constexpr uint64_t wanted = 8192;
-    if (n_tiles == 0 || n_tiles >= 3072) return 0;
-    const uint64_t chunks = 2 * n_primitives / (wanted * backward_chunk) + 1;
-    return static_cast<uint32_t>(chunks) * backward_chunk;
-}
-
 bool launch_blend_backward(const BlendBackwardArgs& a, hipStream_t s) {
     if (a.n_tiles == 0) return true;
-    const dim3 grid(a.n_tiles, a.segment > 0 ? a.n_segment_blocks : 1u);
-    if (a.segment > 0) {
+    const dim3 grid(a.n_tiles, a.checkpoints ? a.n_segment_blocks : 1u);
+    if (a.checkpoints) {
         if (a.abs_grads)
             blend_backward_kernel<true, backward_list_abs, true><<<grid, 64, 0, s>>>(a);
         else

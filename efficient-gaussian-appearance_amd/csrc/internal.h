@@ -143,12 +143,28 @@ struct BlendForwardArgs {
     uint32_t hwc;                  // image layout (H, W, 3)
     uint32_t clamp;                // image clamped to [0, 1] (NaN to 0)
     float4* checkpoints;           // (slots x 192) per segment start: T and colour of every pixel (null: no segments)
-    uint32_t segment;              // instances per segment, a multiple of 32 (0: no segments)
 };
-// Small frames: the backward walks a tile's list in segments, one wave each, from the transmittance and colour that the
-// forward recorded at the segment's start (0: whole lists). Segment k >= 1 of the tile whose instances start at s has
-// the slot s / segment + k: the slots of a frame's segments are distinct and at most (instances) / segment.
-uint32_t instances_per_segment(uint64_t n_primitives, uint32_t n_tiles);
+// Frames of few tiles: the backward walks a tile's list in segments, one wave each, from the transmittance and colour
+// that the forward recorded at the segment's start. Segment k >= 1 of the tile whose instances start at s has the slot
+// s / segment + k: the slots of a frame's segments are distinct and at most (instances) / segment.
+//
+// Segments only where the tiles alone leave most of the GPU's wave slots (four backward waves on each of 1,024 SIMDs)
+// empty. Measured, backward and forward (which records the states and closes its window at a segment's end): 256 tiles of
+// 100 instances 43 -> 18 and 24 -> 26 us; 2,250 tiles of 370 (300k Gaussians at 800 x 533) 133 -> 102 and 83 -> 90 us;
+// 3,350 tiles of 96 64 -> 59 and 32 -> 37 us; 5,382 tiles of 97 101 -> 105 and 45 -> 47 us: the line lies at 3,072 tiles.
+constexpr uint32_t segmented_tiles = 3072;
+// A segment's length: at most 10,923 segments per frame, of whole 32-instance chunks. Short segments cost the forward, long
+// ones leave the backward too few waves: segments of 64, 96, 128 and 160 measured, forward + backward, 97 + 101, 93 + 102, 92 +
+// 105 and 90 + 107 us on 300k Gaussians at 800 x 533 (833k instances: 96 here), and where few of a long list's instances
+// contribute, most segments are blocks that find nothing to do: 20k large Gaussians at 800 x 533 (4.3M instances) 135 us with
+// 512, 166 with 32. It follows the frame's own instance count, which the forward reads on the device and the backward from its
+// frame, and not the buffers' capacity, which depends on the frames before: a frame's gradients are the same bit for bit
+// whatever ran before it.
+constexpr uint32_t segment_chunk_instances = 349525;  // 2^20 / 3
+__host__ __device__ inline uint32_t instances_per_segment(uint32_t n_instances) { return 32u * (n_instances / segment_chunk_instances + 1u); }
+// slots of the segment starts of any frame of at most `capacity` instances (34 MB at most: I instances in segments of
+// 32 c, c = I / 349,525 + 1, have slots up to I / (32 c) < 10,923)
+inline uint64_t segment_slots(uint64_t capacity) { return (capacity < segment_chunk_instances ? capacity : segment_chunk_instances) / 32 + 1; }
 bool launch_blend_forward(const BlendForwardArgs& a, hipStream_t s);
 
 struct BlendBackwardArgs {
@@ -166,8 +182,8 @@ struct BlendBackwardArgs {
     float* inst_grads;             // (I x 9, or I x 12 with abs_grads), emission order (pruning scores: one float per instance)
     uint32_t width, height, grid_w, n_tiles;
     uint32_t abs_grads;            // also reduce |dL/dmean2d| (third densification row)
-    const float4* checkpoints;     // the forward's, with its segment length (segment 0: whole lists)
-    uint32_t segment;
+    const float4* checkpoints;     // the forward's (null: whole lists)
+    uint32_t segment;              // instances_per_segment of the frame
     uint32_t n_segment_blocks;     // blocks per tile; the last one walks every segment from its own on
 };
 bool launch_blend_backward(const BlendBackwardArgs& a, hipStream_t s);

@@ -33,7 +33,7 @@ using torch::autograd::variable_list;
 // steady state a call makes a single allocation.
 class Workspace {
   public:
-    enum Kind { forward = 0, backward = 1, decode = 2 };
+    enum Kind { forward = 0, backward = 1, decode = 2, forward_no_backward = 3 };
 
     Workspace(Kind kind, at::Device device) : key_(kind, device.index()), options_(at::TensorOptions().dtype(at::kByte).device(device)) {
         size_t capacity = 0;
@@ -132,6 +132,7 @@ struct Frame : torch::CustomClassHolder {
     efgs_rasterizer* rasterizer = nullptr;
     Camera camera;
     efgs_frame frame{};
+    std::array<int64_t, 4> counts{};  // primitives, visible primitives, instances, tiles
     std::vector<Tensor> buffers;
     Tensor densification;
     int64_t rows = 0;
@@ -184,15 +185,22 @@ struct Rasterize : torch::autograd::Function<Rasterize> {
         cam.native.bg_color = static_cast<const float*>(cam.background.data_ptr());
         const Tensor image = at::empty({3, cam.native.height, cam.native.width}, at::TensorOptions().dtype(at::kFloat).device(device));
         const efgs_primitives prims = native_primitives(inputs);
+        if (!state->differentiable) {
+            Workspace workspace(Workspace::forward_no_backward, device);
+            check_status(efgs_forward_no_backward(state->rasterizer, &prims, &cam.native, static_cast<float*>(image.data_ptr()), efgs_workspace_alloc,
+                                                  workspace.context(), state->counts.data(), current_stream(device)));
+            workspace.finish();
+            return image;
+        }
         Workspace workspace(Workspace::forward, device);
         check_status(efgs_forward(state->rasterizer, &prims, &cam.native, static_cast<float*>(image.data_ptr()), efgs_workspace_alloc,
                                   workspace.context(), &state->frame, current_stream(device)));
         state->buffers = workspace.finish();
-        if (state->differentiable) {
-            ctx->saved_data["frame"] = c10::IValue::make_capsule(state);
-            ctx->saved_data["mlp_numel"] = mlp_weights.numel();
-            ctx->save_for_backward({image, means, scales, rotations, opacities, precomputed, base, residual, mlp});
-        }
+        const efgs_frame& f = state->frame;
+        state->counts = {f.n_primitives, f.n_visible, f.n_instances, static_cast<int64_t>(f.grid_width) * f.grid_height};
+        ctx->saved_data["frame"] = c10::IValue::make_capsule(state);
+        ctx->saved_data["mlp_numel"] = mlp_weights.numel();
+        ctx->save_for_backward({image, means, scales, rotations, opacities, precomputed, base, residual, mlp});
         return image;
     }
 
@@ -283,8 +291,7 @@ std::pair<Tensor, std::array<int64_t, 4>> diff_rasterize(uintptr_t rasterizer, c
     for (const Tensor* t : {&means, &scales, &rotations, &opacities, &pre, &base_colors, &residual_params, &mlp_weights})
         state->differentiable = state->differentiable || (at::GradMode::is_enabled() && t->requires_grad());
     Tensor image = Rasterize::apply(means, scales, rotations, opacities, pre, base_colors, residual_params, mlp_weights, state);
-    const efgs_frame& f = state->frame;
-    return {std::move(image), {f.n_primitives, f.n_visible, f.n_instances, static_cast<int64_t>(f.grid_width) * f.grid_height}};
+    return {std::move(image), state->counts};
 }
 
 struct NeuralDecode : torch::autograd::Function<NeuralDecode> {

@@ -85,7 +85,7 @@ class FrameViews(ctypes.Structure):
 lib = ctypes.CDLL(LIB_PATH)
 
 EXPORTED = ('efgs_last_error', 'efgs_set_rtc_dirs', 'efgs_rasterizer_create', 'efgs_rasterizer_destroy', 'efgs_set_appearance',
-            'efgs_set_residual_mlp', 'efgs_mlp_param_count', 'efgs_forward', 'efgs_backward', 'efgs_adam_step',
+            'efgs_set_residual_mlp', 'efgs_mlp_param_count', 'efgs_forward', 'efgs_forward_no_backward', 'efgs_backward', 'efgs_adam_step',
             'efgs_get_frame_views', 'efgs_precompile', 'efgs_set_stage_timing', 'efgs_get_stage_times', 'efgs_workspace_alloc',
             'efgs_neural_decode_forward', 'efgs_neural_decode_backward', 'efgs_neural_decode_backward_no_alloc', 'efgs_add_noise', 'efgs_relocation_adjustment', 'efgs_render', 'efgs_update_pruning_scores',
             'efgs_ngsplat_layout', 'efgs_ngsplat_pack')
@@ -106,6 +106,8 @@ lib.efgs_mlp_param_count.restype = ctypes.c_int64
 lib.efgs_mlp_param_count.argtypes = [ctypes.c_void_p]
 lib.efgs_forward.argtypes = [ctypes.c_void_p, ctypes.POINTER(Primitives), ctypes.POINTER(Settings), ctypes.c_void_p, ALLOC_FN,
                              ctypes.c_void_p, ctypes.POINTER(Frame), ctypes.c_void_p]
+lib.efgs_forward_no_backward.argtypes = [ctypes.c_void_p, ctypes.POINTER(Primitives), ctypes.POINTER(Settings), ctypes.c_void_p, ALLOC_FN,
+                                         ctypes.c_void_p, ctypes.POINTER(ctypes.c_int64), ctypes.c_void_p]
 lib.efgs_backward.argtypes = [ctypes.c_void_p, ctypes.POINTER(Primitives), ctypes.POINTER(Settings), ctypes.POINTER(Frame),
                               ctypes.c_void_p, ctypes.c_void_p, ctypes.POINTER(Gradients), ALLOC_FN, ctypes.c_void_p, ctypes.c_void_p]
 lib.efgs_adam_step.argtypes = [ctypes.POINTER(AdamGroup), ctypes.c_int, ctypes.c_void_p]

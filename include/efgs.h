@@ -152,6 +152,12 @@ int efgs_forward(efgs_rasterizer* r, const efgs_primitives* prims, const efgs_se
 int efgs_render(efgs_rasterizer* r, const efgs_primitives* prims, const efgs_settings* settings, float* image, int to_chw, int clamp_output,
                 efgs_alloc_fn alloc, void* alloc_ctx, void* stream);
 
+/* efgs_forward for an image that gets no backward: the same image, without the state that efgs_backward reads (buffers
+ * are dead on return, stream-ordered). counts (optional, 4 entries): primitives, visible primitives, instances, tiles.
+ * No counterpart in the reference (a no-grad diff_rasterize runs its _C.forward). */
+int efgs_forward_no_backward(efgs_rasterizer* r, const efgs_primitives* prims, const efgs_settings* settings, float* image,
+                             efgs_alloc_fn alloc, void* alloc_ctx, int64_t* counts, void* stream);
+
 typedef struct efgs_gradients {
     float* means;                 /* (N, 3) written */
     float* scales;                /* (N, 3) written */
