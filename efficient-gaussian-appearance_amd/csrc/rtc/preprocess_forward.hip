@@ -134,12 +134,15 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v, OP op) {
 
 // exact number of tiles in the tile rectangle that the primitive reaches; first_tiles receives the test results of
 // the rectangle's first mask_tiles tiles (bit i: tile i, row-major). Every lane of the wave must call it.
-// The wave's (primitive, tile) pairs are laid end to end, the primitives in lane order, and tested 64 at a time, one
-// per lane: as many tests as the wave's rectangles hold tiles, where a loop over each lane's own rectangle takes as
-// many steps as the largest of the 64 (and needs a second, cooperative loop for the large ones). With the colour
-// read beside the projection's inputs, against eight tiles per lane and a cooperative step per larger primitive:
-// 10k SH3 Gaussians at 256 x 192 14.1 -> 11.3 us, 150k SV at 1237 x 823 26.9 -> 21.1, 400k SH3 at 1296 x 840 35.9 -> 32.8,
-// 1M neural at 1080p 57.3 -> 51.5.
+// The wave's (primitive, tile) pairs of the rectangles up to coop_tiles tiles are laid end to end, the primitives in lane
+// order, and tested 64 at a time, one per lane: as many tests as the rectangles hold tiles, where a loop over each lane's
+// own rectangle takes as many steps as the largest of the 64. With the colour read beside the projection's inputs,
+// against eight tiles per lane and a cooperative step per larger primitive: 10k SH3 Gaussians at 256 x 192 14.1 -> 11.3
+// us, 150k SV at 1237 x 823 26.9 -> 21.1, 400k SH3 at 1296 x 840 35.9 -> 32.8, 1M neural at 1080p 57.3 -> 51.5.
+// A larger rectangle fills the wave's lanes by itself: the wave tests it alone, 64 tiles per step, its parameters in
+// scalar registers and without the owner search, about half the work of a window step (2k Gaussians of 10,160 tiles at 1080p:
+// 2.9 ms, 5.2 laid end to end; 20k of 213 at 800 x 533 129 and 189 us).
+constexpr uint32_t coop_tiles = 64;
 __device__ inline uint32_t count_touched_tiles(const Projected& pr, uint32_t lane, unsigned char* area, uint32_t& first_tiles) {
 #pragma clang fp contract(off)
     float4* const row_a = reinterpret_cast<float4*>(area);
@@ -147,12 +150,12 @@ __device__ inline uint32_t count_touched_tiles(const Projected& pr, uint32_t lan
     uint32_t* const row_c = reinterpret_cast<uint32_t*>(row_b + 64);
     uint32_t* const marks = row_c + 64;
     const uint32_t bw = pr.tiles.x1 - pr.tiles.x0;
-    const uint32_t cnt = pr.visible ? bw * (pr.tiles.y1 - pr.tiles.y0) : 0u;
+    const uint32_t all = pr.visible ? bw * (pr.tiles.y1 - pr.tiles.y0) : 0u;
+    const uint32_t cnt = all <= coop_tiles ? all : 0u;
     const uint32_t end = wave_inclusive_scan(cnt, [](uint32_t x, uint32_t y) { return x + y; }), start = end - cnt;
     const uint32_t total = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(end), 63));
-    // j / bw for a tile index j < cnt as (j inv) >> 15, exact while cnt bw < 2^15 (inv exceeds 2^15 / bw by at most 1);
-    // a wave with a larger rectangle divides
-    const bool divide = __ballot(cnt * bw >= 32768u || cnt >= 32768u) != 0;
+    // j / bw for a tile index j < cnt as (j inv) >> 15, exact while cnt bw < 2^15 (inv exceeds 2^15 / bw by at most 1)
+    static_assert(coop_tiles * coop_tiles < 1u << 15, "exact for every rectangle of the windows");
     if (cnt > 0) {
         const uint32_t inv = static_cast<uint32_t>(32768.0f * __builtin_amdgcn_rcpf(static_cast<float>(bw))) + 1u;
         row_a[lane] = make_float4(pr.mean2d_x - 0.5f, pr.mean2d_y - 0.5f, pr.conic_x, pr.conic_y);
@@ -172,7 +175,7 @@ __device__ inline uint32_t count_touched_tiles(const Projected& pr, uint32_t lan
         const float4 a = row_a[owner], b = row_b[owner];
         const uint32_t c = row_c[owner], xy = __float_as_uint(b.z);
         const uint32_t j = w0 + lane - __float_as_uint(b.w), w = c & 0xffffu;
-        const uint32_t ty = divide ? j / w : (j * (c >> 16)) >> 15;
+        const uint32_t ty = (j * (c >> 16)) >> 15;
         const uint32_t tx = j - ty * w;
         const bool hit = w0 + lane < total && will_primitive_contribute(a.x, a.y, a.z, a.w, b.x, (xy & 0xffffu) + tx, (xy >> 16) + ty, b.y);
         const uint64_t m = __ballot(hit);
@@ -183,6 +186,26 @@ __device__ inline uint32_t count_touched_tiles(const Projected& pr, uint32_t lan
             if (w0 + lo - start < mask_tiles) first_tiles |= static_cast<uint32_t>(own) << (w0 + lo - start);
         }
         wave_lds_sync();  // the marks are read before the next window's
+    }
+    static_assert(mask_tiles <= 64, "the first step of a large rectangle holds its mask");
+    for (uint64_t coop = __ballot(all > coop_tiles); coop != 0; coop &= coop - 1) {
+        const int src = static_cast<int>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(__ffsll(static_cast<long long>(coop)) - 1)));
+        const auto lane_u = [src](uint32_t v) { return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), src)); };
+        const auto lane_f = [src](float v) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src)); };
+        const uint32_t c_x0 = lane_u(pr.tiles.x0), c_y0 = lane_u(pr.tiles.y0), c_bw = lane_u(bw), c_all = lane_u(all);
+        const float c_mx = lane_f(pr.mean2d_x - 0.5f), c_my = lane_f(pr.mean2d_y - 0.5f);
+        const float c_cx = lane_f(pr.conic_x), c_cy = lane_f(pr.conic_y), c_cz = lane_f(pr.conic_z), c_pt = lane_f(pr.power_threshold);
+        uint32_t hits = 0, first = 0;
+        for (uint32_t base = 0; base < c_all; base += 64) {
+            const uint32_t i = base + lane;
+            const uint64_t m = __ballot(i < c_all && will_primitive_contribute(c_mx, c_my, c_cx, c_cy, c_cz, c_x0 + i % c_bw, c_y0 + i / c_bw, c_pt));
+            if (base == 0) first = static_cast<uint32_t>(m);
+            hits += static_cast<uint32_t>(__popcll(m));
+        }
+        if (lane == static_cast<uint32_t>(src)) {
+            touched = hits;
+            first_tiles = first;
+        }
     }
     return touched;
 }

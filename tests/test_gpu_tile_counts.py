@@ -40,3 +40,28 @@ def test_tile_counts(model, n, width, height, shift):
         b = fw.bounds[vis].astype(np.int64)
         bw = (b[:, 1] + 15) // 16 - b[:, 0] // 16
         assert (bw * bw * ((b[:, 3] + 11) // 12 - b[:, 2] // 12)).max() >= 32768
+
+
+@pytest.mark.parametrize('width,height,shift', [(800, 600, 2.5), (4160, 3180, 1.0)])
+def test_rectangle_limits(width, height, shift):
+    """Rectangles of 32 tiles (the most that emission's mask holds) and 33, of 64 (the most that are tested in the shared
+    windows) and 65, in waves that hold all of these, on a grid of the fused emission and one past it."""
+    import torch
+    from efgs.rasterization import forward_with_frame, frame_views
+    n = 3000
+    scene, app, cam = small_case(model='sh', n=n, width=width, height=height, seed=n, scale_shift=shift)
+    fw = O.render(scene, app, cam)
+    vis = fw.n_touched > 0
+    b = fw.bounds[vis].astype(np.int64)
+    tiles = ((b[:, 1] + 15) // 16 - b[:, 0] // 16) * ((b[:, 3] + 11) // 12 - b[:, 2] // 12)
+    assert {32, 33, 64, 65} <= set(tiles.tolist())
+    dev = torch.device('cuda:0')
+    configure(app)
+    inp = torch_inputs(scene, dev)
+    _, frame, bufs = forward_with_frame(inp['means'], inp['scales'], inp['rotations'], inp['opacities'], settings(cam, dev),
+                                        base_colors=inp['base_colors'], residual_params=inp['residual_params'])
+    torch.cuda.synchronize()
+    v = frame_views(frame)
+    np.testing.assert_array_equal(read_device(bufs, v.n_touched, n, np.uint32), fw.n_touched)
+    check_first_tiles(read_device(bufs, v.records, 12 * n, np.float32).reshape(n, 12)[vis], fw, vis, *cam.grid())
+    check_emission(bufs, v, frame, fw, n)
