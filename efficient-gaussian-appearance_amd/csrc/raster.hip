@@ -63,6 +63,7 @@ __device__ __forceinline__ uint32_t wave_reduce(uint32_t v, OP op) {
 __device__ __forceinline__ uint32_t wave_sum(uint32_t v) { return wave_reduce(v, [](uint32_t x, uint32_t y) { return x + y; }); }
 // a lane's value in every lane; the lane index must be wave-uniform
 __device__ __forceinline__ uint32_t lane_value(uint32_t v, uint32_t src) { return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(src))); }
+__device__ __forceinline__ float lane_value(float v, uint32_t src) { return __uint_as_float(lane_value(__float_as_uint(v), src)); }
 
 __global__ __launch_bounds__(preprocess_block) void compact_visible_kernel(const uint32_t* n_touched, const uint32_t* block_offsets,
                                                                           uint32_t* visible_out, uint32_t* prim_offset, uint32_t n) {
@@ -167,20 +168,28 @@ __device__ __forceinline__ void emit_wave(const CreateInstancesArgs& a, uint32_t
     }
     const uint64_t lanes_below = (1ull << lane) - 1ull;
     uint64_t coop = __ballot(large);
+    if (coop == 0) return;
+    // the large rectangles' records, one per lane and all in flight together (read one by one as each turn came, 20k
+    // Gaussians of 106 tiles at 800 x 533 took 178 us, 168 with them)
+    const uint32_t own = primitive_of(lane);
+    PrimRecord rec{};
+    if (large) rec = a.records[own];
+    const uint32_t bx = __float_as_uint(rec.r2.y), by = __float_as_uint(rec.r2.z);
+    const TileRect t = screen_to_tile_bounds(bx & 0xffffu, bx >> 16, by & 0xffffu, by >> 16);
+    const float power = large ? power_threshold_of(rec.r1.y) : 0.0f;
     while (coop != 0) {
         const uint32_t src = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(__ffsll(static_cast<long long>(coop)) - 1));
         coop &= coop - 1;
-        const uint32_t c_off = lane_value(off, src), c_n = lane_value(n, src), c_p = __builtin_amdgcn_readfirstlane(primitive_of(src));
-        const PrimRecord rec = a.records[c_p];
-        const uint32_t bx = __float_as_uint(rec.r2.y), by = __float_as_uint(rec.r2.z);
-        const TileRect t = screen_to_tile_bounds(bx & 0xffffu, bx >> 16, by & 0xffffu, by >> 16);
-        const uint32_t bw = t.x1 - t.x0, cnt = bw * (t.y1 - t.y0);
-        const float pt = power_threshold_of(rec.r1.y);
+        const uint32_t c_off = lane_value(off, src), c_n = lane_value(n, src), c_p = lane_value(own, src);
+        const uint32_t x0 = lane_value(t.x0, src), y0 = lane_value(t.y0, src);
+        const uint32_t bw = lane_value(t.x1, src) - x0, cnt = bw * (lane_value(t.y1, src) - y0);
+        const float mx = lane_value(rec.r0.x - 0.5f, src), my = lane_value(rec.r0.y - 0.5f, src);
+        const float cx = lane_value(rec.r0.z, src), cy = lane_value(rec.r0.w, src), cz = lane_value(rec.r1.x, src), pt = lane_value(power, src);
         uint32_t k = 0;
         for (uint32_t base = 0; base < cnt; base += 64) {
             const uint32_t j = base + lane;
-            const uint32_t tx = t.x0 + j % bw, ty = t.y0 + j / bw;
-            const bool hit = j < cnt && will_primitive_contribute(rec.r0.x - 0.5f, rec.r0.y - 0.5f, rec.r0.z, rec.r0.w, rec.r1.x, tx, ty, pt);
+            const uint32_t tx = x0 + j % bw, ty = y0 + j / bw;
+            const bool hit = j < cnt && will_primitive_contribute(mx, my, cx, cy, cz, tx, ty, pt);
             const uint64_t m = __ballot(hit);
             const uint32_t pos = k + static_cast<uint32_t>(__popcll(m & lanes_below));
             if (hit && pos < c_n) {
