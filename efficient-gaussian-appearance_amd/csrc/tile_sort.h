@@ -5,7 +5,8 @@
 //                     j < K within a lane, j >= K with the lane at xor distance j / K (128 < n <= 192: a
 //                     128-key and a 64-key network merged by rank);
 //   n > 256           chunks of 256 sorted by the register network; two of them (n <= 512) merged by rank in the
-//                     wave's LDS slab, more by merge passes through the tile's bucket range in global memory.
+//                     wave's LDS slab, more by merge passes of 256 outputs at a time, read from and written to the tile's
+//                     bucket range in global memory.
 #pragma once
 
 #include "internal.h"
@@ -212,12 +213,16 @@ __device__ __forceinline__ uint32_t merge_split(const uint64_t* a, uint32_t na, 
 // Up to 512 keys: both chunks in the slab, a key's position its index in its chunk plus its rank in the other (the
 // 512-key network in the slab that this replaced ran 45 steps of dependent LDS round trips). More: the chunks' keys
 // replace the bucket entries (8 of their 16 bytes each: chunk c's keys end before the entries of chunk c + 1), and
-// merge passes double the sorted length, each lane merging n / 64 consecutive outputs of a pass, between the lower and
-// the upper half of the tile's bucket range (a rank search of every key in every other chunk replaced by log2 passes).
-// Bound by the latency of one wave's dependent steps: 300k Gaussians at 800 x 533 (370 instances per tile on average),
-// forward blend 158 -> 83 us.
+// merge passes double the sorted length, between the lower and the upper half of the tile's bucket range. A pass writes
+// 256 outputs at a time: the two runs' share of them is found by merge path (Odeh, Green et al. 2012: a binary search
+// along the diagonal; a lane per block, 63 blocks at once), read into half of the slab in whole lines while the block
+// before is merged, and each lane merges four consecutive outputs from the slab after a search of its own there. (With
+// n / 64 consecutive outputs per lane read straight from global memory, every key cost a cache line of traffic and a
+// trip to the L2 in turn.) Forward blend, now, with the lanes' own merges, and with the rank search in every other chunk
+// before those: 1,880 instances per tile on 10,800 tiles 0.71, 2.91 and 1.78 ms; 1,890 on 2,250 tiles 187, 484 and 1,007
+// us; 9,100 on 10,800 tiles 5.4, 25.3 and 31.2 ms; 48k in one tile 6.5, 8.1 and 88 ms.
 template <typename KeyT>
-__device__ inline void sort_big_run(uint4* bucket, uint2 r, uint32_t n, uint32_t tile, uint32_t* sorted_inst, KeyT* sorted_keys,
+__device__ __forceinline__ void sort_big_run(uint4* bucket, uint2 r, uint32_t n, uint32_t tile, uint32_t* sorted_inst, KeyT* sorted_keys,
                              const uint32_t* inst_prim, uint32_t* sorted_prim, uint32_t lane, uint64_t* s) {
     constexpr uint32_t K = sort_chunk / 64;
     const uint4* const run = bucket + r.x;
@@ -256,32 +261,66 @@ __device__ inline void sort_big_run(uint4* bucket, uint2 r, uint32_t n, uint32_t
     }
     // (one base pointer and 32-bit positions: n is far below 2^30, a run's range of 2 n keys fits)
     uint32_t src = 0, dst = n;
-    const uint32_t per = (n + 63u) / 64u;
-    for (uint32_t width = sort_chunk; width < n; width *= 2) {
+    for (uint32_t width = sort_chunk; width < n; width *= 2) {  // (widths are powers of two: a block lies in one pair of runs)
         const bool last = 2 * width >= n;
-        uint32_t x = min(lane * per, n);
-        const uint32_t x_end = min(x + per, n);
-        while (x < x_end) {  // the lane's outputs, pair of runs by pair of runs
-            const uint32_t p0 = x & ~(2 * width - 1u), p1 = min(p0 + 2 * width, n);  // (widths are powers of two)
-            const uint32_t na = min(width, n - p0);
-            uint32_t ia = src + p0, ib = ia + na;  // next keys of the two runs
-            const uint32_t ea = ib, eb = src + p1;
-            const uint32_t split = merge_split(keys + ia, na, keys + ib, eb - ib, x - p0);
-            ia += split;
-            ib += x - p0 - split;
-            uint64_t ka = ia < ea ? keys[ia] : ~0ull, kb = ib < eb ? keys[ib] : ~0ull;
-            for (const uint32_t end = min(x_end, p1); x < end; x++) {
-                const bool from_a = ka < kb;  // (a run past its end yields the largest key, which no instance has)
-                const uint64_t key = from_a ? ka : kb;
-                if (from_a) {
-                    ia++;
-                    ka = ia < ea ? keys[ia] : ~0ull;
-                } else {
-                    ib++;
-                    kb = ib < eb ? keys[ib] : ~0ull;
+        const auto pair_of = [&](uint32_t x, uint32_t& p0, uint32_t& na, uint32_t& nb) {
+            p0 = x & ~(2 * width - 1u);
+            na = min(width, n - p0);
+            nb = min(2 * width, n - p0) - na;
+        };
+        for (uint32_t x_batch = 0; x_batch < n; x_batch += 63u * sort_chunk) {
+            // lane l: the first run's share of its pair's outputs up to the start of block l
+            uint32_t split;
+            {
+                const uint32_t x = min(x_batch + lane * sort_chunk, n);
+                uint32_t p0, na, nb;
+                pair_of(x, p0, na, nb);
+                split = merge_split(keys + src + p0, na, keys + src + p0 + na, nb, x - p0);
+            }
+            uint64_t next[K];  // the block's keys: `ca` of the first run, then the second's, element t in lane t % 64
+            const auto load = [&](uint32_t block, uint32_t& count, uint32_t& ca) {
+                const uint32_t x = x_batch + block * sort_chunk;
+                uint32_t p0, na, nb;
+                pair_of(x, p0, na, nb);
+                count = min(sort_chunk, p0 + na + nb - x);
+                const uint32_t a0 = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(split), static_cast<int>(block)));
+                const uint32_t end = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(split), static_cast<int>(block + 1u)));
+                ca = (x + count == p0 + na + nb ? na : end) - a0;
+                const uint32_t first = src + p0 + a0, second = src + p0 + na + (x - p0 - a0) - ca;
+#pragma unroll
+                for (uint32_t i = 0; i < K; i++) {
+                    const uint32_t t = lane + 64u * i;
+                    next[i] = t < count ? keys[(t < ca ? first : second) + t] : ~0ull;
                 }
-                if (last) o.put(x, key);
-                else keys[dst + x] = key;
+            };
+            const uint32_t n_blocks = min(63u, (n - x_batch + sort_chunk - 1u) / sort_chunk);
+            uint32_t count, ca;
+            load(0, count, ca);
+            for (uint32_t block = 0; block < n_blocks; block++) {
+                uint64_t* const m = s + (block & 1u) * sort_chunk;  // (the half that the block before last left)
+#pragma unroll
+                for (uint32_t i = 0; i < K; i++) m[lane + 64u * i] = next[i];
+                const uint32_t c = count, c_a = ca, x = x_batch + block * sort_chunk + K * lane;
+                if (block + 1u < n_blocks) load(block + 1u, count, ca);
+                wave_lds_fence();
+                if (K * lane < c) {
+                    uint32_t ia = merge_split(m, c_a, m + c_a, c - c_a, K * lane), ib = K * lane - ia + c_a;
+                    uint64_t ka = ia < c_a ? m[ia] : ~0ull, kb = ib < c ? m[ib] : ~0ull;
+                    for (uint32_t i = 0; i < K && K * lane + i < c; i++) {
+                        const bool from_a = ka < kb;  // (a run past its end yields the largest key, which no instance has)
+                        const uint64_t key = from_a ? ka : kb;
+                        if (from_a) {
+                            ia++;
+                            ka = ia < c_a ? m[ia] : ~0ull;
+                        } else {
+                            ib++;
+                            kb = ib < c ? m[ib] : ~0ull;
+                        }
+                        if (last) o.put(x + i, key);
+                        else keys[dst + x + i] = key;
+                    }
+                }
+                wave_lds_fence();
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");

@@ -36,3 +36,9 @@ def test_run_lengths(n):
     prims = read_device(bufs, v.instance_primitive, n, np.uint32)
     np.testing.assert_array_equal(prims[slots], order)
     assert not read_device(bufs, v.tile_sorted_keys, n, np.uint16).any()
+
+
+@pytest.mark.parametrize('n', [16128, 16129, 16385, 40000])
+def test_long_runs(n):
+    """Runs past one batch of 63 merge blocks (16,128 outputs), with a last block of one key."""
+    test_run_lengths(n)
