@@ -9,7 +9,6 @@
 // _C.backward).
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/csrc/autograd/custom_function.h>
-#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/utils/pybind.h>
 #include <torch/extension.h>
 
@@ -139,18 +138,22 @@ struct Frame : torch::CustomClassHolder {
     bool differentiable = false;
 };
 
-// gradients of a backward that is itself being differentiated: their own gradient raises, as for a function marked
-// once_differentiable
-variable_list once_differentiable(variable_list grads, const variable_list& upstream) {
-    if (!at::GradMode::is_enabled()) return grads;
-    bool requires_grad = false;
-    for (const Tensor& g : upstream) requires_grad = requires_grad || (g.defined() && g.requires_grad());
-    if (!requires_grad) return grads;
-    variable_list fake;
-    for (Tensor& g : grads) fake.push_back(g.defined() ? g.detach().requires_grad_(true) : g);
-    auto error = std::make_shared<torch::autograd::DelayedError>(
-        "trying to differentiate twice a function that was marked with @once_differentiable", static_cast<int64_t>(fake.size()));
-    return (*error)(std::move(fake));
+// The gradients of a backward that is itself being differentiated (create_graph with an upstream that requires a
+// gradient) hang on the upstream by an identity whose own backward raises: the kernels have no second derivatives, and a
+// graph without this edge would give zeros for them. The message is the one that Python autograd functions marked
+// once_differentiable give, which programs may look for.
+struct FirstOrderOnly : torch::autograd::Function<FirstOrderOnly> {
+    static Tensor forward(AutogradContext*, const Tensor& /*upstream*/, const Tensor& grad) { return grad.variable_data(); }  // (no view: it may be changed in place)
+    static variable_list backward(AutogradContext*, variable_list) {
+        TORCH_CHECK(false, "trying to differentiate twice a function that was marked with @once_differentiable");
+    }
+};
+
+variable_list first_order_only(variable_list grads, const Tensor& upstream) {
+    if (at::GradMode::is_enabled() && upstream.requires_grad())
+        for (Tensor& g : grads)
+            if (g.defined()) g = FirstOrderOnly::apply(upstream, g);
+    return grads;
 }
 
 struct Rasterize : torch::autograd::Function<Rasterize> {
@@ -211,7 +214,7 @@ struct Rasterize : torch::autograd::Function<Rasterize> {
             at::NoGradGuard no_grad;
             grads = gradients(ctx, saved, upstream[0]);
         }
-        return once_differentiable(std::move(grads), upstream);
+        return first_order_only(std::move(grads), upstream[0]);
     }
 
     static variable_list gradients(AutogradContext* ctx, const variable_list& saved, const Tensor& upstream) {
@@ -319,7 +322,7 @@ struct NeuralDecode : torch::autograd::Function<NeuralDecode> {
             at::NoGradGuard no_grad;
             grads = gradients(ctx, saved, upstream[0]);
         }
-        return once_differentiable(std::move(grads), upstream);
+        return first_order_only(std::move(grads), upstream[0]);
     }
 
     static variable_list gradients(AutogradContext* ctx, const variable_list& saved, const Tensor& upstream) {

@@ -95,3 +95,19 @@ def test_refusals(case):
     with pytest.raises(ValueError, match='image gradient'):
         image = render()
         image.grad_fn(grad[:, 1:])
+
+
+def test_gradients_of_gradients(case):
+    """With an upstream that requires a gradient, the gradients hold the same values, may be changed in place, and raise when
+    they are differentiated; with one that does not, they require no gradient."""
+    torch, render, inp, grad = case
+    want = _grads(torch, render(), inp, grad)
+    up = grad.clone().requires_grad_(True)
+    got = torch.autograd.grad(render(), [inp[k] for k in NAMES], up, create_graph=True)
+    assert _same(want, got) and all(g.requires_grad for g in got)
+    got[0].mul_(2.0)
+    assert bool((got[0] == 2.0 * want[0]).all())
+    for g in got:
+        with pytest.raises(RuntimeError, match='differentiate twice'):
+            g.sum().backward(retain_graph=True)
+    assert not any(g.requires_grad for g in torch.autograd.grad(render(), [inp[k] for k in NAMES], grad, create_graph=True))
