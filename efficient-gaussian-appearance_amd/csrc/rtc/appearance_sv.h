@@ -86,14 +86,6 @@ __device__ __forceinline__ float3 sv_color(const SvState& v) {
     return make_float3(wr * v.r, wr * v.g, wr * v.b);
 }
 
-template <int RES_ACT>
-__device__ inline float3 sv_residual(const float* p, float3 d, uint32_t sites) {
-    if (sites == 0) return make_float3(0.0f, 0.0f, 0.0f);
-    SvState v;
-    sv_add_sites<RES_ACT>(v, p, d, sites);
-    return sv_color(v);
-}
-
 // writes dL/d(site parameters) of the active sites and returns dL/dmean through the view direction. A site's
 // parameters are read before its gradients are written, and no later step reads them, so gp may be p0 itself.
 template <int RES_ACT>

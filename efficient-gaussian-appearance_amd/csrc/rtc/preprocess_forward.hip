@@ -327,7 +327,6 @@ extern "C" __global__ __launch_bounds__(256, 4) void EFGS_KERNEL_NAME(efgs::Prep
         const float3 cam = make_float3(a.cam.cam_position[0], a.cam.cam_position[1], a.cam.cam_position[2]);
         float norm_rcp;
         const float3 d = view_direction(pr.mean, cam, norm_rcp);
-        const float* rp = a.residual + static_cast<size_t>(p) * residual_params;
         float3 res = make_float3(0.0f, 0.0f, 0.0f);
 #if EFGS_MODEL == 5
         // The chunk's visible primitives, compacted in thread order into the staging rows, run the MLP on as few
@@ -344,7 +343,7 @@ extern "C" __global__ __launch_bounds__(256, 4) void EFGS_KERNEL_NAME(efgs::Prep
             if (visible) {
                 float x[nn::INP];
                 const float base[3] = {pr.color.x, pr.color.y, pr.color.z};
-                nn::mlp_input(rp, base, d, a.cam.degree, x);
+                nn::mlp_input(a.residual + static_cast<size_t>(p) * residual_params, base, d, a.cam.degree, x);
                 nn::stage_input_row(stage, x, row);
             }
             __syncthreads();  // rows staged (and every read of wave_counts done)
@@ -360,6 +359,7 @@ extern "C" __global__ __launch_bounds__(256, 4) void EFGS_KERNEL_NAME(efgs::Prep
         }
 #endif
 #if EFGS_MODEL >= 1 && EFGS_MODEL <= 4
+        static_assert(ForwardRows::staged || EFGS_N_UNITS == 0, "every layout with units is staged");
         if constexpr (ForwardRows::staged) {
             const uint32_t p0 = chunk * preprocess_block + wave_u * 64u;
             const float* const row = rows + lane * row_ld;
@@ -387,16 +387,6 @@ extern "C" __global__ __launch_bounds__(256, 4) void EFGS_KERNEL_NAME(efgs::Prep
             }
 #if EFGS_MODEL == 2
             if (visible && a.cam.degree > 0) res = sv_color(sv);
-#endif
-        } else if (visible) {
-#if EFGS_MODEL == 1
-            res = sh_residual<EFGS_RES_ACT>(rp, d, a.cam.degree);
-#elif EFGS_MODEL == 2
-            res = sv_residual<EFGS_RES_ACT>(rp, d, a.cam.degree);
-#elif EFGS_MODEL == 3
-            res = lobe_residual<EFGS_RES_ACT, false>(rp, d, a.cam.degree);
-#elif EFGS_MODEL == 4
-            res = lobe_residual<EFGS_RES_ACT, true>(rp, d, a.cam.degree);
 #endif
         }
 #endif

@@ -12,7 +12,7 @@ constexpr uint32_t residual_params = EFGS_MODEL == 0 ? 0u : params_per_unit * EF
 // a wave's lines fall out of the L1 and the L2 between the loads that share them (400k SH3 primitives: 271 MB read
 // for 94 MB of rows). SH takes its coefficients in one pass, SV and the lobe models up to MAX_UNITS units per pass:
 // four lobes are 128 (144) bytes of a row, where passes of two lobes fetched every 128-byte line twice (NASG forward on
-// 1M primitives: 488 MB for 312 MB). A layout above 63 floats per pass (WHOLE_ROW: per row) reads its rows directly.
+// 1M primitives: 488 MB for 312 MB). A WHOLE_ROW layout of more than 63 floats reads its rows directly.
 // Preprocess times before and after (the block-wide staging, respectively direct reads, of single floats with index
 // arithmetic per element): NASG on 1M at 1080p 120 -> 90 us forward, 181 -> 142 us backward; SH3 on 400k 66 -> 36 us
 // forward; SV on 150k 31.0 -> 30.6 and 37.9 -> 35.0 us.
