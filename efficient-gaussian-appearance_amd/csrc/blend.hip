@@ -8,9 +8,10 @@
 // Front-to-back compositing, alpha = o exp2(min(q, 0)) with the conic pre-scaled by -log2(e)/2 and the hardware
 // exp2 (v_exp_f32, as the reference's fast-math exp2f), alpha < 1/255 skipped, stop at T < 1e-4; stores the image,
 // final T and last-contributor index per pixel and the per-tile maximum (an inference render stores only the
-// image, in CHW or HWC layout, optionally clamped). No per-bucket checkpoints.
+// image, in CHW or HWC layout, optionally clamped). In frames of fewer than 3,072 tiles that get a backward also the pixels'
+// transmittance and colour at the start of every list segment (see instances_per_segment).
 //
-// Backward: one wave per tile, sixteen 4x3 pixel groups, three pixels per lane (see blend_backward_kernel). Every
+// Backward: one wave per tile (in the segmented frames, per segment of a tile's list), sixteen 4x3 pixel groups, three pixels per lane (see blend_backward_kernel). Every
 // pixel replays its forward walk (the evaluation is shared and compiled with -ffp-contract=off, so T and every
 // skip decision are reproduced bit-exactly; which pixels evaluate a Gaussian differs from the forward only where
 // its alpha is below 1/255, outside its screen rectangle) and forms the reference's per-pixel terms; the
@@ -137,7 +138,7 @@ __device__ __forceinline__ float rows_reduce1(float v) {
     return swap16_add(w, w);
 }
 
-// Backward, one wave per tile. Lane l serves column k = l >> 4 of pixel group i = l & 15, a 4x3 block of the tile
+// Backward, one wave per tile (or per segment of its list, from the state that the forward recorded there). Lane l serves column k = l >> 4 of pixel group i = l & 15, a 4x3 block of the tile
 // (columns 4 (i & 3) + 0..3, rows 3 (i >> 2) + 0..2), and that column's three pixels. Every pixel replays its forward
 // walk (alpha bit-identical, the decisions are the forward's) and forms, branch-free (zero where it skips the
 // Gaussian), h = -alpha dL/dalpha with dL/dalpha = T (c . g) - (A - g_bg) / max(1 - alpha, eps), A = (colour still

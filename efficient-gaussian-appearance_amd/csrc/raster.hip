@@ -170,7 +170,7 @@ __device__ __forceinline__ void emit_wave(const CreateInstancesArgs& a, uint32_t
     uint64_t coop = __ballot(large);
     if (coop == 0) return;
     // the large rectangles' records, one per lane and all in flight together (read one by one as each turn came, 20k
-    // Gaussians of 106 tiles at 800 x 533 took 178 us, 168 with them)
+    // Gaussians of 106 tiles at 800 x 533 took 178 us, 166 with them)
     const uint32_t own = primitive_of(lane);
     PrimRecord rec{};
     if (large) rec = a.records[own];
@@ -582,7 +582,7 @@ __global__ __launch_bounds__(256) void tile_buckets_kernel(const KeyT* keys, con
     const uint32_t n_chunks = (n_instances + bucket_chunk - 1u) / bucket_chunk;
     if (block >= n_chunks) return;  // (block-uniform: the grid covers a bound on I)
     // XCD-aware chunk: the hardware deals workgroups to the 8 XCDs round robin (workgroup w on XCD w % 8, so bucket
-    // block b on XCD (b + 1) % 8); the blocks of one XCD take one contiguous run of the chunks, so the table rows of
+    // block b on XCD (b + lead) % 8); the blocks of one XCD take one contiguous run of the chunks, so the table rows of
     // a segment (whose instances are contiguous) are fetched into one XCD's L2 instead of all eight
     const uint32_t xcd = block % 8u, per = n_chunks / 8u, extra = n_chunks % 8u;
     const uint32_t chunk = xcd * per + min(xcd, extra) + block / 8u;

@@ -35,7 +35,8 @@ constexpr float min_alpha = 1.0f / 255.0f;
 //   r1 = (conic.z, opacity, color.r, color.g)
 //   r2 = (color.b, bits(x_min | x_max << 16), bits(y_min | y_max << 16), bits(first-tiles mask))
 // where bit j of the mask (j < n_sequential_tiles) records whether tile j of the primitive's tile rectangle (row-major order)
-// passes the contribution test, as the preprocess counted it
+// passes the contribution test, as the preprocess counted it: the low bits of the mask that emission reads (below), which
+// no kernel reads here and which the parity tests compare with the oracle
 struct PrimRecord {
     float4 r0, r1, r2;
 };
