@@ -1159,6 +1159,15 @@ int efgs_get_frame_views(const efgs_frame* frame, efgs_frame_views* v) {
     return EFGS_OK;
 }
 
+int efgs_get_frame_tile_views(const efgs_frame* frame, const uint32_t** tile_rects, const uint32_t** tile_order) {
+    if (!frame || !tile_rects || !tile_order) return fail(EFGS_ERR_INVALID_ARGUMENT, "null argument");
+    const uint32_t n_tiles = static_cast<uint32_t>(frame->grid_width) * static_cast<uint32_t>(frame->grid_height);
+    *tile_rects = reinterpret_cast<const uint32_t*>(
+        PrimitiveLayout::carve(static_cast<char*>(frame->primitive_buffers), static_cast<uint32_t>(frame->n_primitives)).tile_rects);
+    *tile_order = TileLayout::carve(static_cast<char*>(frame->tile_buffers), n_tiles).order;
+    return EFGS_OK;
+}
+
 namespace {
 
 int check_decode(const efgs_rasterizer* r, int64_t n, const float* features, const float* base, const float* dirs,

@@ -43,13 +43,6 @@ class Frame(ctypes.Structure):
                 ('instance_capacity', ctypes.c_int64), ('grid_width', ctypes.c_int32), ('grid_height', ctypes.c_int32), ('key_bytes', ctypes.c_int32), ('model', ctypes.c_int32)]
 
 
-class Gradients(ctypes.Structure):
-    _fields_ = [('means', ctypes.c_void_p), ('scales', ctypes.c_void_p), ('rotations', ctypes.c_void_p),
-                ('opacities', ctypes.c_void_p), ('precomputed_colors', ctypes.c_void_p), ('base_colors', ctypes.c_void_p),
-                ('residual_params', ctypes.c_void_p), ('mlp_weights', ctypes.c_void_p), ('densification_info', ctypes.c_void_p),
-                ('densification_rows', ctypes.c_int)]
-
-
 class AdamGroup(ctypes.Structure):
     _fields_ = [('grad', ctypes.c_void_p), ('param', ctypes.c_void_p), ('exp_avg', ctypes.c_void_p),
                 ('exp_avg_sq', ctypes.c_void_p), ('n_elements', ctypes.c_int64), ('step', ctypes.c_int64),
@@ -86,7 +79,7 @@ lib = ctypes.CDLL(LIB_PATH)
 
 EXPORTED = ('efgs_last_error', 'efgs_set_rtc_dirs', 'efgs_rasterizer_create', 'efgs_rasterizer_destroy', 'efgs_set_appearance',
             'efgs_set_residual_mlp', 'efgs_mlp_param_count', 'efgs_forward', 'efgs_forward_no_backward', 'efgs_backward', 'efgs_adam_step',
-            'efgs_get_frame_views', 'efgs_precompile', 'efgs_set_stage_timing', 'efgs_get_stage_times', 'efgs_workspace_alloc',
+            'efgs_get_frame_views', 'efgs_get_frame_tile_views', 'efgs_precompile', 'efgs_set_stage_timing', 'efgs_get_stage_times', 'efgs_workspace_alloc',
             'efgs_neural_decode_forward', 'efgs_neural_decode_backward', 'efgs_neural_decode_backward_no_alloc', 'efgs_add_noise', 'efgs_relocation_adjustment', 'efgs_render', 'efgs_update_pruning_scores',
             'efgs_ngsplat_layout', 'efgs_ngsplat_pack')
 
@@ -108,10 +101,9 @@ lib.efgs_forward.argtypes = [ctypes.c_void_p, ctypes.POINTER(Primitives), ctypes
                              ctypes.c_void_p, ctypes.POINTER(Frame), ctypes.c_void_p]
 lib.efgs_forward_no_backward.argtypes = [ctypes.c_void_p, ctypes.POINTER(Primitives), ctypes.POINTER(Settings), ctypes.c_void_p, ALLOC_FN,
                                          ctypes.c_void_p, ctypes.POINTER(ctypes.c_int64), ctypes.c_void_p]
-lib.efgs_backward.argtypes = [ctypes.c_void_p, ctypes.POINTER(Primitives), ctypes.POINTER(Settings), ctypes.POINTER(Frame),
-                              ctypes.c_void_p, ctypes.c_void_p, ctypes.POINTER(Gradients), ALLOC_FN, ctypes.c_void_p, ctypes.c_void_p]
 lib.efgs_adam_step.argtypes = [ctypes.POINTER(AdamGroup), ctypes.c_int, ctypes.c_void_p]
 lib.efgs_get_frame_views.argtypes = [ctypes.POINTER(Frame), ctypes.POINTER(FrameViews)]
+lib.efgs_get_frame_tile_views.argtypes = [ctypes.POINTER(Frame), ctypes.POINTER(ctypes.c_void_p), ctypes.POINTER(ctypes.c_void_p)]
 lib.efgs_precompile.argtypes = [ctypes.c_void_p, ctypes.c_char_p]
 lib.efgs_set_stage_timing.argtypes = [ctypes.c_void_p, ctypes.c_int]
 lib.efgs_workspace_alloc.restype = ctypes.c_void_p

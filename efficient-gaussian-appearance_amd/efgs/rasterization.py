@@ -293,6 +293,13 @@ def frame_views(frame: _lib.Frame) -> _lib.FrameViews:
     return v
 
 
+def frame_tile_views(frame: _lib.Frame) -> tuple[int, int]:
+    """Device pointers to a frame's tile rectangles with their masks and to the blends' tile order (likewise)."""
+    rects, order = ctypes.c_void_p(), ctypes.c_void_p()
+    check(lib.efgs_get_frame_tile_views(ctypes.byref(frame), ctypes.byref(rects), ctypes.byref(order)))
+    return rects.value, order.value
+
+
 def forward_with_frame(means, scales, rotations, opacities, rasterizer_settings: RasterizerSettings, precomputed_colors=None,
                        base_colors=None, residual_params=None, mlp_weights=None):
     """Forward pass returning (image, frame, buffers): the frame and the buffers that back it, for inspection."""

@@ -313,7 +313,7 @@ int efgs_neural_decode_backward_no_alloc(efgs_rasterizer* r, int64_t n, const fl
 typedef struct efgs_frame_views {
     const uint32_t* n_touched;        /* (N) 0 = culled */
     const uint32_t* depth_keys;       /* (N) float bits of the view depth (valid where n_touched > 0) */
-    const float* records;             /* (N x 12) mean2d xy, conic xyz, opacity, rgb, packed bounds, pad */
+    const float* records;             /* (N x 12) mean2d xy, conic xyz, opacity, rgb, packed bounds, first 8 bits of the tile mask */
     const uint32_t* visible_prims;       /* (V) the visible primitives in index order */
     const uint32_t* prim_offset;         /* (N) first emission slot of each visible primitive (exclusive scan of
                                             n_touched in index order) */
@@ -327,6 +327,10 @@ typedef struct efgs_frame_views {
     const uint32_t* counters;            /* (8) V, I, instance-count mismatches, min and max visible depth key, reserved */
 } efgs_frame_views;
 int efgs_get_frame_views(const efgs_frame* frame, efgs_frame_views* views);
+/* Two more, likewise: tile_rects (N x 2, visible primitives: first tile's x | y << 13 | width << 26 of the tile rectangle, the
+ * width 63 above 32 tiles; bit j: reaches tile j of the rectangle, row-major, the first 32) and tile_order (T: the tiles in
+ * the order in which the blends take them, heaviest class first). */
+int efgs_get_frame_tile_views(const efgs_frame* frame, const uint32_t** tile_rects, const uint32_t** tile_order);
 
 /* Compiles the preprocess kernels of the current configuration into the hipRTC cache for `arch` (e.g.
  * "gfx950") without using a device (no counterpart in the reference; build step). */

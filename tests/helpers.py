@@ -191,14 +191,15 @@ def check_emission(bufs, v, frame, fw, n: int) -> None:
     np.testing.assert_array_equal(read_device(bufs, v.instance_primitive, I, np.uint32), fw.inst_prims[order])
 
 
-# tiles of a primitive's rectangle whose test results the preprocess records in the record's spare word
+# tiles of a primitive's rectangle whose test results the record's spare word holds (the low bits of the mask that instance
+# emission reads)
 SEQUENTIAL_TILES = 8
 
 
 def check_first_tiles(rec: np.ndarray, fw, vis: np.ndarray, grid_w: int, grid_h: int) -> None:
     """The record's spare word (column 11): bit j (j < SEQUENTIAL_TILES) set exactly when tile j of the primitive's
-    tile rectangle (row-major) is one of the tiles the oracle emits for it (the preprocess's tile-test results that
-    instance emission reads instead of testing again). rec: the device records of the visible primitives."""
+    tile rectangle (row-major) is one of the tiles the oracle emits for it. rec: the device records of the visible
+    primitives."""
     prims = np.nonzero(vis)[0]
     b = fw.bounds[vis].astype(np.int64)
     x0, x1 = b[:, 0] // 16, (b[:, 1] + 15) // 16
@@ -215,3 +216,25 @@ def check_first_tiles(rec: np.ndarray, fw, vis: np.ndarray, grid_w: int, grid_h:
         hit = (j < cnt) & (emitted[pos] == code) if len(emitted) else np.zeros(len(prims), bool)
         expected |= hit.astype(np.uint32) << np.uint32(j)
     np.testing.assert_array_equal(rec[:, 11].view(np.uint32), expected)
+
+
+def check_tile_rects(rects: np.ndarray, fw, vis: np.ndarray, grid_w: int) -> None:
+    """What instance emission reads of the visible primitives: the tile rectangle's first tile and width (63 above 32 tiles) and,
+    up to 32 tiles, the mask whose bit j is set exactly when the oracle emits tile j of the rectangle (row-major). rects: the
+    device's (x | y << 13 | width << 26, mask) of the visible primitives."""
+    prims = np.nonzero(vis)[0]
+    b = fw.bounds[vis].astype(np.int64)
+    x0, y0 = b[:, 0] // 16, b[:, 2] // 12
+    bw = (b[:, 1] + 15) // 16 - x0
+    cnt = bw * ((b[:, 3] + 11) // 12 - y0)
+    small = cnt <= 32
+    np.testing.assert_array_equal(rects[:, 0], (x0 | y0 << 13 | np.where(small, bw, 63) << 26).astype(np.uint32))
+    row = np.full(len(fw.n_touched), -1, np.int64)
+    row[prims] = np.arange(len(prims))
+    i = row[fw.inst_prims.astype(np.int64)]
+    key = fw.inst_keys.astype(np.int64)
+    j = (key // grid_w - y0[i]) * bw[i] + key % grid_w - x0[i]
+    keep = small[i]
+    expected = np.zeros(len(prims), np.uint64)
+    np.bitwise_or.at(expected, i[keep], np.uint64(1) << j[keep].astype(np.uint64))
+    np.testing.assert_array_equal(rects[small, 1], expected[small].astype(np.uint32))
