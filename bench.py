@@ -53,9 +53,9 @@ STAGE_KERNELS = {
     # not timed, and create_instances_fused_kernel carries the compaction's bytes)
     'compact': 'scan_block_counts_kernel + compact_visible_kernel',
     'create_instances': 'create_instances_fused_kernel',
-    'tile_offsets': 'tile_column_scan_kernel',  # (the tile order's runs are placed by an extra block of tile_buckets_kernel)
-    'tile_buckets': 'tile_buckets_kernel',
-    'tile_sort': 'tile_ranges_kernel',  # (the tiles' runs are sorted by blend_forward_kernel, before its walk)
+    'tile_offsets': 'tile_column_scan_kernel',
+    'tile_buckets': 'tile_buckets_kernel',  # (up to 16,384 tiles its first blocks write the tiles' ranges and order)
+    'tile_sort': 'tile_ranges_kernel',  # (larger grids; the tiles' runs are sorted by blend_forward_kernel, before its walk)
     'blend_forward': 'blend_forward_kernel',
     'blend_backward': 'blend_backward_kernel',
     'preprocess_backward': 'preprocess_backward_<model>',
@@ -105,18 +105,21 @@ def algorithmic(stage: str, N: int, V: int, I: int, T: int, P: int, R: int, mlp_
     its LDS: V*48 + I*6 for that one kernel, and no compaction stage), tile ranges T*8; the ordering by (tile, depth) -- the reference's depth sort and
     offset scan (V*24) and tile sort (I*12) -- split into the bucketing (I*6: tile key in, emission index
     out) and the per-tile sort (I*6 + V*24), which the forward blend runs before its walk; the tiles' ranges and
-    order T*24 (three words in, two out); blend forward I*48 + P*20 (+ the sort); blend backward P*32 + I*76;
+    order T*24 (three words in, two out; up to 16,384 tiles part of the bucketing, which writes them, and no kernel of their
+    own); blend forward I*48 + P*20 (+ the sort); blend backward P*32 + I*76;
     preprocess backward V*(110+R) + N*(56+R), for the neural model split into the geometry kernel
     (V*110 + N*56 + (N-V)*R: culled primitives' zero latent gradients) and the MLP kernel (V*2R: latents in,
     latent gradients out); Adam 28 B per element. MLP FLOPs: forward V*F, backward (input and weight
     gradients, forward recomputed) 2*V*F, F = unpadded forward FLOPs per primitive."""
+    ranges = T * 24
+    ranges_in_buckets = T <= 16384
     table = {
         'preprocess_forward': (N * (60 + R) + V * 44, V * mlp_fwd_flops),
         'compact': (V * 8, 0),
         'create_instances': (V * (48 if compaction_fused else 40) + I * 6, 0),
         'tile_offsets': (T * 8, 0),
-        'tile_buckets': (I * 6, 0),
-        'tile_sort': (T * 24, 0),
+        'tile_buckets': (I * 6 + (ranges if ranges_in_buckets else 0), 0),
+        'tile_sort': (0 if ranges_in_buckets else ranges, 0),
         'blend_forward': (I * 48 + P * 20 + I * 6 + V * 24, 0),
         'blend_backward': (P * 32 + I * 76, 0),
         'preprocess_backward': ((V * 110 + N * 56 + (N - V) * R, 0) if mlp_fwd_flops

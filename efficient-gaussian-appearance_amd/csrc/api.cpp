@@ -802,9 +802,11 @@ int forward_impl(efgs_rasterizer* r, const efgs_primitives* prims, const efgs_se
                                  tl.ranges, n_tiles, s))
             return EFGS_ERR_HIP;
         t.end(s);
-        t.begin(EFGS_STAGE_TILE_SORT, s);
-        if (!launch_tile_ranges(ts, tl.ranges, max_instances, n_tiles, s)) return EFGS_ERR_HIP;
-        t.end(s);
+        if (tile_ranges_kernel_needed(max_instances, n_tiles)) {
+            t.begin(EFGS_STAGE_TILE_SORT, s);
+            if (!launch_tile_ranges(ts, tl.ranges, n_tiles, s)) return EFGS_ERR_HIP;
+            t.end(s);
+        }
 
         BlendForwardArgs b;
         b.ranges = tl.ranges;

@@ -117,8 +117,9 @@ bool launch_tile_buckets(const TileBinning& plan, const void* keys, int key_byte
                          const uint32_t* table, const uint32_t* local_rank, const TileScan& ts, uint4* bucket, uint32_t max_instances,
                          uint2* ranges, uint32_t n_tiles, hipStream_t s);
 // per tile: [start, end) into ranges and its place in the blends' tile order (the runs are sorted by the forward blend);
-// nothing where launch_tile_buckets has written them
-bool launch_tile_ranges(const TileScan& ts, uint2* ranges, uint32_t max_instances, uint32_t n_tiles, hipStream_t s);
+// not needed where launch_tile_buckets has written them
+bool tile_ranges_kernel_needed(uint32_t max_instances, uint32_t n_tiles);
+bool launch_tile_ranges(const TileScan& ts, uint2* ranges, uint32_t n_tiles, hipStream_t s);
 bool launch_reduce_partials(const float* partials, uint32_t n_blocks, uint32_t n_params, float* out, hipStream_t s);
 
 struct BlendForwardArgs {

@@ -787,8 +787,11 @@ bool launch_tile_buckets(const TileBinning& plan, const void* keys, int key_byte
     return true;
 }
 
-bool launch_tile_ranges(const TileScan& ts, uint2* ranges, uint32_t max_instances, uint32_t n_tiles, hipStream_t s) {
-    if (n_tiles == 0 || (max_instances > 0 && div_up(n_tiles, scan_tiles) <= order_direct_blocks)) return true;
+bool tile_ranges_kernel_needed(uint32_t max_instances, uint32_t n_tiles) {
+    return n_tiles > 0 && (max_instances == 0 || div_up(n_tiles, scan_tiles) > order_direct_blocks);
+}
+
+bool launch_tile_ranges(const TileScan& ts, uint2* ranges, uint32_t n_tiles, hipStream_t s) {
     tile_ranges_kernel<<<div_up(n_tiles, 256), 256, 0, s>>>(ts.totals, ts.block_sums, ts.local_start, ts.order_runs, ts.order_rank, ts.order,
                                                             ts.counters, ranges, n_tiles);
     EFGS_HIP_CHECK(hipGetLastError());

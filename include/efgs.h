@@ -346,9 +346,10 @@ enum {
     EFGS_STAGE_COUNTER_READ = 2,       /* (V, I) device-to-host read and stream synchronisation */
     EFGS_STAGE_CREATE_INSTANCES = 3,   /* (tile, primitive) instances at their emission slots, per-tile counts */
     EFGS_STAGE_TILE_OFFSETS = 4,       /* scan of the per-tile counts: tile ranges */
-    EFGS_STAGE_TILE_BUCKETS = 5,       /* instances into their tiles' ranges */
-    EFGS_STAGE_TILE_SORT = 6,          /* the tiles' ranges and the blends' tile order (the per-tile (depth, primitive)
-                                          sort itself runs inside the forward blend, EFGS_STAGE_BLEND_FORWARD) */
+    EFGS_STAGE_TILE_BUCKETS = 5,       /* instances into their tiles' ranges; on grids of up to 16,384 tiles also the tiles'
+                                          ranges and the blends' tile order */
+    EFGS_STAGE_TILE_SORT = 6,          /* larger grids (and frames without instances): the ranges and the order (the per-tile
+                                          (depth, primitive) sort itself runs inside the forward blend) */
     EFGS_STAGE_BLEND_FORWARD = 7,
     EFGS_STAGE_BLEND_BACKWARD = 8,
     EFGS_STAGE_PREPROCESS_BACKWARD = 9,
