@@ -30,12 +30,12 @@ constexpr float lobe_log2e = 1.44269504088896340736f, lobe_ln2 = 0.6931471805599
 // e^4, values 0.90 and 0.98), because of three things that cost a few instructions each: tanh and sech of small angles
 // by polynomial (as 1 - 2 u^2 / (1 + u^2) at all angles, tanh has an absolute error of 6e-8 where it should have a
 // relative one, and angle gradients were 1.4 to 1.6 times as far off), sech x instead of sqrt(1 - tanh^2 x) for large
-// ones, and lobe_view below. With them NASG on 1M Gaussians at 1080p takes 94 us forward and 149.5 us backward, 90 and 144.5
-// without (213 us backward on the library's functions).
+// ones, and lobe_view below. With them NASG on 1M Gaussians at 1080p takes 95 us forward and 148 us backward, 90 and 145
+// without (119 and 213 on the library's functions).
 
 // tanh x and sech x = sqrt(1 - tanh^2 x). |x| < 0.7: polynomials in x^2 (x + x^3 P and 1 + x^2 Q; P and Q fitted for the least
-// largest relative error of the result, 2e-8); above, from u = exp(-|x|): 1 - 2 u^2 / (1 + u^2) with the sign of x, and
-// 2 u / (1 + u^2). (Up to 0.5 with one coefficient less: the same time, errors 3 to 6 % larger.)
+// largest relative error of the result, 2e-8); above, from u = exp(-|x|): sech x = 2 u / (1 + u^2) and tanh |x| =
+// 1 - u sech x. (Up to 0.5 with one coefficient less: the same time, errors 3 to 6 % larger.)
 __device__ __forceinline__ float lobe_tanh(float x, float& sech) {
     const float z = x * x;
     float p = __builtin_fmaf(z, -5.13866186e-3f, 2.00919697e-2f);
@@ -47,11 +47,10 @@ __device__ __forceinline__ float lobe_tanh(float x, float& sech) {
     q = __builtin_fmaf(z, q, 2.08265854e-1f);
     q = __builtin_fmaf(z, q, -4.99997688e-1f);
     const float u = __builtin_amdgcn_exp2f(-lobe_log2e * fabsf(x));
-    const float u2 = u * u;
-    const float d = __builtin_amdgcn_rcpf(1.0f + u2);
+    const float s = (u + u) * __builtin_amdgcn_rcpf(__builtin_fmaf(u, u, 1.0f));
     const bool small = fabsf(x) < 0.7f;
-    sech = small ? __builtin_fmaf(z, q, 1.0f) : 2.0f * u * d;
-    return small ? __builtin_fmaf(x * z, p, x) : __builtin_copysignf(__builtin_fmaf(-2.0f * u2, d, 1.0f), x);
+    sech = small ? __builtin_fmaf(z, q, 1.0f) : s;
+    return small ? __builtin_fmaf(x * z, p, x) : __builtin_copysignf(__builtin_fmaf(-u, s, 1.0f), x);
 }
 
 // exp x with the rounding of x log2 e compensated (x clamped to the range of finite, normal results; NaN: the largest)
@@ -222,13 +221,15 @@ __device__ inline float3 lobe_residual_backward(const float* p, float3 gc, float
         gd.x += gvx * f.x.x + gvz * f.z.x;
         gd.y += gvx * f.x.y + gvz * f.z.y;
         gd.z += gvx * f.x.z + gvz * f.z.z;
-        const float dst = -f.ct * __builtin_amdgcn_rcpf(f.st), dsp = -f.cp * __builtin_amdgcn_rcpf(f.sp), dsu = -f.cu * __builtin_amdgcn_rcpf(f.su);
-        const float gct = gxx * (f.cp * f.cu - dst * f.su) + gxy * (dst * f.cp * f.cu + f.su) + gzx * f.sp + gzy * dst * f.sp;
-        const float gcp = gxx * f.ct * f.cu + gxy * f.st * f.cu - gxz * dsp * f.cu + gzx * f.ct * dsp + gzy * f.st * dsp + gzz;
-        const float gcu = gxx * (f.ct * f.cp - f.st * dsu) + gxy * (f.st * f.cp + f.ct * dsu) - gxz * f.sp;
-        gp[0] = fabsf(th) >= lobe_cos_limit ? 0.0f : gct * (f.st * f.st);
-        gp[1] = fabsf(tp) >= lobe_cos_limit ? 0.0f : gcp * (f.sp * f.sp);
-        gp[2] = fabsf(tu) >= lobe_cos_limit ? 0.0f : gcu * (f.su * f.su);
+        // d cos = sin^2 d raw for each angle, and d sin = -(cos / sin) d cos: one sin of the sin^2 cancels the quotient (the
+        // three reciprocals and products of the quotients 152 -> 148 us)
+        const float cc = f.cp * f.cu, q = gxx * f.ct + gxy * f.st;
+        const float gt = f.st * (gxx * cc + gxy * f.su + gzx * f.sp) - f.ct * (gxy * cc - gxx * f.su + gzy * f.sp);
+        const float gph = f.sp * (q * f.cu + gzz) - f.cp * (gzx * f.ct + gzy * f.st - gxz * f.cu);
+        const float gta = f.su * (q * f.cp - gxz * f.sp) - f.cu * (gxy * f.ct - gxx * f.st);
+        gp[0] = fabsf(th) >= lobe_cos_limit ? 0.0f : gt * f.st;
+        gp[1] = fabsf(tp) >= lobe_cos_limit ? 0.0f : gph * f.sp;
+        gp[2] = fabsf(tu) >= lobe_cos_limit ? 0.0f : gta * f.su;
     }
     return direction_grad_to_mean(gd, d, norm_rcp);
 }
