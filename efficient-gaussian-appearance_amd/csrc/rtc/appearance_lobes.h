@@ -31,7 +31,7 @@ constexpr float lobe_log2e = 1.44269504088896340736f, lobe_ln2 = 0.6931471805599
 // by polynomial (as 1 - 2 u^2 / (1 + u^2) at all angles, tanh has an absolute error of 6e-8 where it should have a
 // relative one, and angle gradients were 1.4 to 1.6 times as far off), sech x instead of sqrt(1 - tanh^2 x) for large
 // ones, and lobe_view below. With them NASG on 1M Gaussians at 1080p takes 95 us forward and 148 us backward, 90 and 145
-// without (119 and 213 on the library's functions).
+// without (213 us backward on the library's functions, with the row staging of the time).
 
 // tanh x and sech x = sqrt(1 - tanh^2 x). |x| < 0.7: polynomials in x^2 (x + x^3 P and 1 + x^2 Q; P and Q fitted for the least
 // largest relative error of the result, 2e-8); above, from u = exp(-|x|): sech x = 2 u / (1 + u^2) and tanh |x| =
