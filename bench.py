@@ -903,7 +903,7 @@ def main() -> None:
 def headline_line(args, r: dict, cpu: dict | None, port: dict | None) -> dict:
     """The bench's JSON line. `value` = W * H / t, t = the HIP-event time of the K timed steps (one pair of events
     around all of them, device synchronisations on both sides) divided by K: the rasterizer's forward and backward,
-    BASELINE.md's headline; `ms_per_step` = t; `wall_ms_per_step` = host wall time of the same K steps divided by K;
+    the reference's headline; `ms_per_step` = t; `wall_ms_per_step` = host wall time of the same K steps divided by K;
     `step_ms_quartiles` = the spread of K more steps, each between its own pair of events (which adds ~10 us per
     step); `gpu_idle_us_per_step` = t minus the kernel time of one steady-state step of the committed kernel trace of
     this command (no kernel running on the GPU)."""
